@@ -699,7 +699,7 @@ static hipError_t prepare_fast() {
 }
 
 template <typename T, int N, int TX, int NT, int IO, bool LINES, class RL, int XM, int WPE>
-static int launch_fast_multi(const MultiGroup *g, int ng, long long tiles, hipStream_t st) {
+static int launch_fast_multi(const MultiGroup *g, int ng, long long tiles, int, size_t, hipStream_t st) {
   using C = FastCfg<T, N, TX, NT, LINES, RL, XM>;
   const long long nb = xcd_grid(tiles);
   if (nb <= 0) return D2DHIP_SUCCESS;

@@ -13,6 +13,7 @@ namespace d2dhip {
 struct FastVariant {
   int rb = 8;      // bytes per real (8 FP64, 4 FP32)
   int mf = 0;      // 1: split-BF16 radix-16 passes on the matrix cores
+  int mixed = 0;   // > 0: any length (mixed_impl.h); shape and radices from mixed_shape
   int io = 0;      // IO_C2C / IO_R2C / IO_C2R
   int lines = 0;   // 1: contiguous lines (x axis), 0: strided columns
   int n = 0;       // FFT length
@@ -22,8 +23,10 @@ struct FastVariant {
   std::vector<int> radices;
   int (*launch)(const AxisDesc *dd, const AxisDesc &h, const AxisIo &io, hipStream_t st) = nullptr;
   hipError_t (*prepare)() = nullptr;
-  // the same kernel over the tiles of several grids (MultiGroup list)
-  int (*launch_multi)(const MultiGroup *g, int ng, long long tiles, hipStream_t st) = nullptr;
+  // the same kernel over the tiles of several grids (MultiGroup list); block
+  // size and LDS of the widest grid, for the kernels of any length
+  int (*launch_multi)(const MultiGroup *g, int ng, long long tiles, int nthreads, size_t lds,
+                      hipStream_t st) = nullptr;
   hipError_t (*prepare_multi)() = nullptr;
   const char *name = "";
 };
@@ -43,6 +46,11 @@ struct PersistKind {
 const std::vector<PersistKind> &persist_kinds(int rb);
 int batch_fast_prepare(int rb, size_t lds, int *blocks_per_cu);
 int launch_batch_fast(int rb, const BatchQueue &q, int blocks, size_t lds, hipStream_t st);
+// The kernels of any length (mixed_impl.h); whether one of them runs length
+// n; and the tile and radix schedule that it takes (C0 tile-level columns).
+std::vector<FastVariant> mixed_variants();
+bool mixed_runs(const FastVariant &v, int n);
+bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &radices, AxisShape &s);
 // The split-BF16 matrix-core variants (mfma_kernels.hip).
 std::vector<FastVariant> mf_variants();
 

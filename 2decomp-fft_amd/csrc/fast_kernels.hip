@@ -181,7 +181,7 @@ int launch_batch_fast(int rb, const BatchQueue &q, int blocks, size_t lds, hipSt
 
 // The registered variants, in candidate order (the first able to run a stage
 // is its default): the parts compiled in fast_variants_*.hip, then the
-// matrix-core kernels.
+// matrix-core kernels, then the kernels of any length.
 std::vector<FastVariant> fast_variants_a();
 std::vector<FastVariant> fast_variants_b();
 std::vector<FastVariant> fast_variants_c();
@@ -197,6 +197,7 @@ const std::vector<FastVariant> &fast_registry() {
       r.insert(r.end(), v.begin(), v.end());
     }
     for (const FastVariant &v : mf_variants()) r.push_back(v);
+    for (const FastVariant &v : mixed_variants()) r.push_back(v);
     return r;
   }();
   return reg;

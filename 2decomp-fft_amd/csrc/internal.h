@@ -110,6 +110,9 @@ struct AxisDesc {
   // IO_DTT4 stages exp(-i pi (4j+1) / (4 dtt_len)), j < n, then
   // exp(-i pi k / dtt_len), k < n (n = dtt_len / 2)
   const void *dtw;
+  // Stages of the mixed kernels (any length): threads that share a tile
+  // column, block size and LDS bytes of a launch.
+  int rows, nthreads, lds_bytes;
 };
 
 #ifdef __HIPCC__  // (a host compiler, for the host-only sanitizer build, skips these)
@@ -211,6 +214,7 @@ struct AxisShape {
   int nthreads = 64;
   size_t lds_bytes = 0;
   int ldj = 1, ldt = 1;
+  int rows = 0;  // mixed kernels: threads per tile column
 };
 
 // Per-axis plan: the radix schedule and twiddles of one FFT length.

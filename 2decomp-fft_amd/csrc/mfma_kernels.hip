@@ -796,7 +796,7 @@ static hipError_t prepare_mf() {
 }
 
 template <int N, int TX, int NT, int IO, bool LINES, class RL, int XM, int WPE, int SW>
-static int launch_mf_multi(const MultiGroup *g, int ng, long long tiles, hipStream_t st) {
+static int launch_mf_multi(const MultiGroup *g, int ng, long long tiles, int, size_t, hipStream_t st) {
   using S = MfShape<N, TX, NT, IO, LINES, RL, XM>;
   const long long nb = xcd_grid(tiles);
   if (nb <= 0) return D2DHIP_SUCCESS;

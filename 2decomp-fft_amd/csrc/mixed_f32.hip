@@ -1,0 +1,8 @@
+// mixed_f32.hip -- the FP32 kernels of any length (mixed_impl.h).
+#include "mixed_impl.h"
+
+namespace d2dhip {
+
+std::vector<FastVariant> mixed_variants_f32() { return {D2D_MIXED_ALL(float)}; }
+
+}  // namespace d2dhip

@@ -1,0 +1,487 @@
+// mixed_impl.h -- axis stages of any length with factors 2-17 (gfx950).
+//
+// The specialised kernels (fast_impl.h) fix the length at compile time and
+// the general kernel (fft_kernels.hip) calls one non-inlined function per
+// pass, which costs it 248 VGPRs (2 waves per SIMD) and callee-saved
+// registers spilled around every call.  Here the radix of a pass is a
+// compile-time case of a uniform switch and everything else (length, tile,
+// rows) is read from the descriptor, so one kernel serves every length at
+// 4 waves per SIMD with no calls and no spills.
+//
+// A workgroup owns a tile of TX columns of n points; `rows` threads share a
+// column and take butterflies row, row + rows, ... of every pass, at most 16
+// values each.  Strided columns put consecutive threads on consecutive tile
+// columns (one run of 128 bytes or more per point); contiguous lines put
+// them on consecutive points of a line.  The first pass reads HBM, the last
+// writes HBM, those in between exchange through LDS; real transforms pair
+// two real columns as the general kernel does.
+//
+// Measured against the general kernel on 0.8 GB stages, FP64 TB/s of the bytes
+// read and written once (columns c2c / lines r2c / lines c2r):
+//   n = 100  2.0 / 2.7 / 2.3 -> 5.2 / 5.5 / 5.1
+//   n = 405  1.9 / 3.0 / 2.4 -> 4.4 / 4.7 / 4.6
+//   n = 1000 1.3 / 2.0 / 1.6 -> 3.9 / 4.9 / 4.9
+// What bounds it: up to 600 points the HBM rate of the access pattern; longer
+// columns the workgroups per CU, since a tile of 8 columns takes over half
+// of the LDS.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "codelets.h"
+#include "fast_kernels.h"
+#include "internal.h"
+
+namespace d2dhip {
+
+namespace {
+
+// Butterflies of radix R that a lane takes per pass: one, or as many as make
+// 10 values (at most 4).
+constexpr int mx_nb(int r) { return r > 5 ? 1 : (10 / r < 4 ? 10 / r : 4); }
+
+// Radices by kernel class: 0 the codelets that fit 128 VGPRs in FP64 at 1024
+// threads, 1 the large primes too (512 threads).
+template <int CLS, class F>
+__device__ __forceinline__ void radix_case(int r, F &&f) {
+  switch (r) {
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 15: f(std::integral_constant<int, 15>{}); break;
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    default:
+      if constexpr (CLS == 1) {
+        if (r == 11) f(std::integral_constant<int, 11>{});
+        else if (r == 13) f(std::integral_constant<int, 13>{});
+        else if (r == 17) f(std::integral_constant<int, 17>{});
+      }
+  }
+}
+
+// w / n and w % n by the reciprocal, corrected to exact (0 <= w < 2^23).
+__device__ __forceinline__ void est_divmod(int w, int n, float inv, int &q, int &r) {
+  q = (int)((float)w * inv);
+  r = w - q * n;
+  if (r < 0) {
+    --q;
+    r += n;
+  } else if (r >= n) {
+    ++q;
+    r -= n;
+  }
+}
+
+template <typename T, int IO, bool LINES, int CLS, bool PK>
+__device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out, int conj,
+                                           long long tile) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  cpx<T> *lds = reinterpret_cast<cpx<T> *>(lds_raw);
+  constexpr bool PAIRED = IO == IO_R2C || IO == IO_C2R;
+  const int n = d->n, TX = d->TX, lg = d->log2TX, rows = d->rows, np = d->npass;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const long long tiles0 = d->tiles0;
+  const long long c1 = tile / tiles0;
+  const long long c0b = (tile - c1 * tiles0) * TX;
+  int t, row;
+  if constexpr (LINES) {
+    est_divmod(tid, rows, 1.0f / (float)rows, t, row);
+  } else {
+    t = tid & (TX - 1);
+    row = tid >> lg;
+  }
+  const long long c0 = c0b + t;
+  const long long ca = PAIRED ? 2 * c0 : c0;  // first (real) column of the lane
+  // lanes without a column or a row take no butterfly (they keep to the barriers)
+  if (t >= TX || row >= rows || ca >= (PAIRED ? d->C0r : d->C0)) row = 1 << 24;
+  const bool two = !PAIRED || ca + 1 < d->C0r;
+  const long long sji = d->in_sj, sjo = d->out_sj;
+  const long long in_base = (IO == IO_R2C ? ca : c0) * d->in_s0 + c1 * d->in_s1 +
+                            (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->in_b0 : 0);
+  const long long out_base = (IO == IO_C2R ? ca : c0) * d->out_s0 + c1 * d->out_s1 +
+                             (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->out_b0 : 0);
+  const void *tw = d->tw;
+  // LDS: [point][column] for strided columns; [line][point] with one pad
+  // point in 17 for contiguous lines, whose first exchange writes with the
+  // stride of the first radix
+  const int ldt = d->ldt;
+  auto A = [&](int j, int tt) __attribute__((always_inline)) {
+    return LINES ? j + (j >> 4) + tt * ldt : (j << lg) + tt;
+  };
+
+  // ---- pieces of a pass ------------------------------------------------------
+  // values of the first pass (and whole transforms of one pass) from HBM
+  auto load = [&](auto rc, auto &v) __attribute__((always_inline)) {
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    const int nb = n / R;
+    const long long step = (long long)nb * sji;
+    if constexpr (IO == IO_R2C) {
+      // adjacent columns whose pairs are aligned: one load per pair
+      const bool vec = !LINES && d->in_s0 == 1 && ((sji | d->in_s1) & 1) == 0 &&
+                       ((unsigned long long)in & (sizeof(cpx<T>) - 1)) == 0;
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          const long long o = in_base + (long long)b * sji;
+          if (vec && two) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) v[q * R + s] = gload<T>(in, (o + s * step) >> 1);
+          } else {
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              v[q * R + s].x = gload_r<T>(in, o + s * step);
+              v[q * R + s].y = two ? gload_r<T>(in, o + s * step + d->in_s0) : T(0);
+            }
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          const long long o = in_base + (long long)b * sji;
+          if (PK && d->packj >= 2) {
+#pragma unroll
+            for (int s0 = 0; s0 < R; s0 += 4) {  // four table reads, then their loads
+              long long off[4];
+#pragma unroll
+              for (int s = s0; s < R && s < s0 + 4; ++s) off[s - s0] = packj_offset(d, b + s * nb, c1);
+#pragma unroll
+              for (int s = s0; s < R && s < s0 + 4; ++s)
+                v[q * R + s] = gload<T>(in, o + s * step + off[s - s0]);
+            }
+          } else {
+#pragma unroll
+            for (int s = 0; s < R; ++s) v[q * R + s] = gload<T>(in, o + s * step);
+          }
+          if (conj) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) v[q * R + s].y = -v[q * R + s].y;
+          }
+        }
+      }
+    }
+  };
+  // outputs j = b + s * (n / R) of the last pass to HBM
+  auto store = [&](auto rc, auto &v) __attribute__((always_inline)) {
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    const int nb = n / R;
+    const long long step = (long long)nb * sjo;
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const int b = row + q * rows;
+      if (b < nb) {
+        const long long o = out_base + (long long)b * sjo;
+        if constexpr (IO == IO_C2R) {  // the pre-phase stored conj(Z): z = conj(result)
+#pragma unroll
+          for (int s = 0; s < R; ++s) {
+            gstore_r<T>(out, o + s * step, v[q * R + s].x);
+            if (two) gstore_r<T>(out, o + s * step + d->out_s0, -v[q * R + s].y);
+          }
+        } else {
+          if (conj) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) v[q * R + s].y = -v[q * R + s].y;
+          }
+          if (PK && (d->packj & 1)) {
+            const long long *tab = d->packj == 1 ? d->pack : d->pack2;
+#pragma unroll
+            for (int s0 = 0; s0 < R; s0 += 4) {
+              long long off[4];
+#pragma unroll
+              for (int s = s0; s < R && s < s0 + 4; ++s) off[s - s0] = packj_offset_in(tab, b + s * nb, c1);
+#pragma unroll
+              for (int s = s0; s < R && s < s0 + 4; ++s)
+                gstore<T>(out, o + s * step + off[s - s0], v[q * R + s]);
+            }
+          } else {
+#pragma unroll
+            for (int s = 0; s < R; ++s) gstore<T>(out, o + s * step, v[q * R + s]);
+          }
+        }
+      }
+    }
+  };
+  // inputs j = b + s * (n / R) of a pass from LDS
+  auto lds_read = [&](auto rc, auto &v, int nb, int row_, int rows_, int t_) __attribute__((always_inline)) {
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const int b = row_ + q * rows_;
+      if (b < nb) {
+#pragma unroll
+        for (int s = 0; s < R; ++s) v[q * R + s] = lds[A(b + s * nb, t_)];
+      }
+    }
+  };
+
+  // ---- inputs ------------------------------------------------------------------
+  const int nh = d->nh;
+  const float inv_nh = 1.0f / (float)nh;
+  if constexpr (IO == IO_C2R) {
+    // conj(Z) of the merged half spectra, all n points, into LDS; the loads
+    // of four points of both columns are in flight together
+    constexpr int U = 4;
+    const int total = TX * nh;
+    for (int w0 = tid; w0 < total; w0 += U * nthr) {
+      cpx<T> a[U], b[U];
+      int kk[U], tt[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int w = w0 + u * nthr;
+        kk[u] = -1;
+        tt[u] = 0;
+        a[u] = b[u] = cpx<T>{T(0), T(0)};
+        if (w < total) {
+          if constexpr (LINES) {
+            est_divmod(w, nh, inv_nh, tt[u], kk[u]);
+          } else {
+            tt[u] = w & (TX - 1);
+            kk[u] = w >> lg;
+          }
+          const long long cc = 2 * (c0b + tt[u]);
+          long long ia = cc * d->in_s0 + c1 * d->in_s1 + (long long)kk[u] * sji;
+          long long ib = ia + d->in_s0;
+          if (LINES && d->npack) {  // receive-buffer order, or the blocked layout
+            ia = pack_index(d, kk[u], cc + c1 * d->pack_l1);
+            ib = pack_index(d, kk[u], cc + 1 + c1 * d->pack_l1);
+          }
+          if (cc < d->C0r) a[u] = gload<T>(in, ia);
+          if (cc + 1 < d->C0r) b[u] = gload<T>(in, ib);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = kk[u];
+        if (k >= 0) {
+          if (k == 0 || 2 * k == n) a[u].y = b[u].y = T(0);
+          lds[A(k, tt[u])] = cpx<T>{a[u].x - b[u].y, -(a[u].y + b[u].x)};
+          if (k > 0 && 2 * k < n) lds[A(n - k, tt[u])] = cpx<T>{a[u].x + b[u].y, a[u].y - b[u].x};
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  // ---- passes --------------------------------------------------------------------
+  constexpr bool HBM_IN = IO != IO_C2R, HBM_OUT = IO != IO_R2C;
+  if (HBM_IN && HBM_OUT && np == 1) {
+    radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      cpx<T> v[NB * R];
+      load(rc, v);
+      if (row < rows) dft<T, R>(v);  // n == R: one butterfly per column
+      store(rc, v);
+    });
+    return;
+  }
+  int p = 0;
+  if constexpr (HBM_IN) {
+    radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      const int nb = n / R;
+      cpx<T> v[NB * R];
+      load(rc, v);
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          dft<T, R>(&v[q * R]);
+#pragma unroll
+          for (int s = 0; s < R; ++s) lds[A(b * R + s, t)] = v[q * R + s];
+        }
+      }
+    });
+    __syncthreads();
+    p = 1;
+  }
+  const int pmid = HBM_OUT ? np - 1 : np;
+  for (; p < pmid; ++p) {
+    const int L = d->pass[p].L, tw_off = d->pass[p].tw_off;
+    const float invL = d->pass[p].invL;
+    // a zero the compiler cannot see through: it would otherwise hoist the
+    // loop-invariant address parts of every radix's case out of the loop, far
+    // more than there are registers (430 bytes of spill per lane)
+    int zero;
+    asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+    const int n_ = n + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
+    radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      const int nb = n_ / R;
+      cpx<T> v[NB * R];
+      lds_read(rc, v, nb, row_, rows_, t_);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row_ + q * rows_;
+        if (b < nb) {
+          int g, k;
+          est_divmod(b, L, invL, g, k);
+          if (L > 1) {
+#pragma unroll
+            for (int s = 1; s < R; ++s)
+              v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + k * (R - 1) + (s - 1)));
+          }
+          dft<T, R>(&v[q * R]);
+          const int jb = g * L * R + k;
+#pragma unroll
+          for (int s = 0; s < R; ++s) lds[A(jb + s * L, t_)] = v[q * R + s];
+        }
+      }
+    });
+    __syncthreads();
+  }
+  if constexpr (HBM_OUT) {
+    const int tw_off = d->pass[np - 1].tw_off;
+    radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      const int nb = n / R;  // = L: every butterfly of the last pass is its own k
+      cpx<T> v[NB * R];
+      lds_read(rc, v, nb, row, rows, t);
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          if (nb > 1) {
+#pragma unroll
+            for (int s = 1; s < R; ++s)
+              v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + b * (R - 1) + (s - 1)));
+          }
+          dft<T, R>(&v[q * R]);
+        }
+      }
+      store(rc, v);
+    });
+  } else {
+    // A[k] = (Z[k] + conj Z[n-k]) / 2 and B[k] = (Z[k] - conj Z[n-k]) / (2i)
+    const T half = T(0.5);
+    const int total = TX * nh;
+    for (int w = tid; w < total; w += nthr) {
+      int tt, k;
+      if constexpr (LINES) {
+        est_divmod(w, nh, inv_nh, tt, k);
+      } else {
+        tt = w & (TX - 1);
+        k = w >> lg;
+      }
+      const long long cc = 2 * (c0b + tt);
+      if (cc < d->C0r) {
+        const cpx<T> zk = lds[A(k, tt)], zm = lds[A(k == 0 ? 0 : n - k, tt)];
+        long long oa = cc * d->out_s0 + c1 * d->out_s1 + (long long)k * sjo;
+        long long ob = oa + d->out_s0;
+        if (LINES && d->npack) {  // send-buffer order, or the blocked layout
+          oa = pack_index(d, k, cc + c1 * d->pack_l1);
+          ob = pack_index(d, k, cc + 1 + c1 * d->pack_l1);
+        }
+        gstore<T>(out, oa, cpx<T>{(zk.x + zm.x) * half, (zk.y - zm.y) * half});
+        if (cc + 1 < d->C0r) gstore<T>(out, ob, cpx<T>{(zk.y + zm.y) * half, (zm.x - zk.x) * half});
+      }
+    }
+  }
+}
+
+// Threads a workgroup may have, and the waves per SIMD its registers leave
+// room for.
+constexpr int mx_threads(int cls) { return cls == 0 ? 1024 : 512; }
+template <typename T>
+constexpr int mx_wpe(int cls) {
+  return cls == 0 ? (sizeof(T) == 8 ? 4 : 6) : (sizeof(T) == 8 ? 2 : 4);
+}
+
+// One grid (ng = 0: the stage of the arguments), or the tiles of several
+// grids (the same code, so that a batch's results equal the plans' own).
+template <typename T, int IO, bool LINES, int CLS, bool PK>
+__global__ void __launch_bounds__(mx_threads(CLS)) __attribute__((amdgpu_waves_per_eu(mx_wpe<T>(CLS))))
+    mixed_kernel(const AxisDesc *__restrict__ d, const void *in, void *out, int conj,
+                 const MultiGroup *__restrict__ g, int ng, long long tiles) {
+  long long it = xcd_tile((long long)blockIdx.x + (long long)blockIdx.y * gridDim.x, tiles);
+  if (it >= tiles) return;  // whole block, before any barrier
+  if (ng > 0) {
+    const int gi = find_multi_group(g, ng, it);
+    d = g[gi].d;
+    in = g[gi].in;
+    out = g[gi].out;
+    conj = g[gi].conj;
+    it -= g[gi].tile0;
+  }
+  mixed_tile<T, IO, LINES, CLS, PK>(desc_ptr(d), in, out, conj, it);
+}
+
+template <typename T, int IO, bool LINES, int CLS, bool PK>
+int mixed_go(const AxisDesc *dd, const AxisIo &io, const MultiGroup *g, int ng, long long tiles, int nt,
+             size_t lds, hipStream_t st) {
+  const long long nb = xcd_grid(tiles);
+  if (nb <= 0) return D2DHIP_SUCCESS;
+  const long long gx = nb < (1LL << 20) ? nb : (1LL << 20);
+  const long long gy = (nb + gx - 1) / gx;
+  if (gy > 65535) return set_error(D2DHIP_ERR_UNSUPPORTED, "axis stage has too many tiles");
+  hipLaunchKernelGGL((mixed_kernel<T, IO, LINES, CLS, PK>), dim3((unsigned)gx, (unsigned)gy), dim3(nt), lds,
+                     st, dd, io.in, io.out, io.conj, g, ng, tiles);
+  return hip_check(hipGetLastError(), "mixed_kernel launch");
+}
+
+template <typename T, int IO, bool LINES, int CLS>
+int mixed_launch(const AxisDesc *dd, const AxisDesc &h, const AxisIo &io, hipStream_t st) {
+  const long long tiles = (long long)h.tiles0 * h.C1;
+  if constexpr (IO == IO_C2C && !LINES) {
+    if (h.packj) return mixed_go<T, IO, LINES, CLS, true>(dd, io, nullptr, 0, tiles, h.nthreads, h.lds_bytes, st);
+  }
+  return mixed_go<T, IO, LINES, CLS, false>(dd, io, nullptr, 0, tiles, h.nthreads, h.lds_bytes, st);
+}
+
+template <typename T, int IO, bool LINES, int CLS>
+int mixed_launch_multi(const MultiGroup *g, int ng, long long tiles, int nt, size_t lds, hipStream_t st) {
+  const AxisIo io = {nullptr, nullptr, 0};
+  return mixed_go<T, IO, LINES, CLS, false>(nullptr, io, g, ng, tiles, nt, lds, st);
+}
+
+constexpr int kMaxLds = 160 * 1024;
+
+template <typename T, int IO, bool LINES, int CLS>
+hipError_t mixed_prepare() {
+  hipError_t e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, false>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+  if constexpr (IO == IO_C2C && !LINES) {
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, true>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+  }
+  return e;
+}
+
+template <typename T, int IO, bool LINES, int CLS>
+FastVariant mixed_variant(const char *name) {
+  FastVariant v;
+  v.rb = (int)sizeof(T);
+  v.io = IO;
+  v.lines = LINES ? 1 : 0;
+  v.mixed = 1 + CLS;
+  v.launch = &mixed_launch<T, IO, LINES, CLS>;
+  v.prepare = &mixed_prepare<T, IO, LINES, CLS>;
+  v.launch_multi = &mixed_launch_multi<T, IO, LINES, CLS>;
+  v.prepare_multi = &mixed_prepare<T, IO, LINES, CLS>;
+  v.name = name;
+  return v;
+}
+
+// c2c, r2c and c2r, strided columns and contiguous lines, both classes
+#define D2D_MIXED(T, IO, LINES, TAG)                               \
+  mixed_variant<T, IO, LINES, 0>(#T " mixed " TAG),                \
+      mixed_variant<T, IO, LINES, 1>(#T " mixed " TAG " primes")
+#define D2D_MIXED_ALL(T)                                                   \
+  D2D_MIXED(T, IO_C2C, false, "c2c"), D2D_MIXED(T, IO_C2C, true, "c2c"),   \
+  D2D_MIXED(T, IO_R2C, false, "r2c"), D2D_MIXED(T, IO_R2C, true, "r2c"),   \
+  D2D_MIXED(T, IO_C2R, false, "c2r"), D2D_MIXED(T, IO_C2R, true, "c2r")
+
+}  // namespace
+
+}  // namespace d2dhip

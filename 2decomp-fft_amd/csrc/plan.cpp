@@ -458,7 +458,11 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   const FastVariant *fv = (c >= 0) ? g.cands[c] : nullptr;
   const BlueTables *bt = nullptr;
   int st;
-  if (fv) {
+  if (fv && fv->mixed) {
+    const long long C0 = g.io == IO_C2C ? g.C0r : (g.C0r + 1) / 2;
+    if (!mixed_shape(*fv, g.n, C0, radices, s))
+      return set_error(D2DHIP_ERR_UNSUPPORTED, "mixed kernel: length not covered");
+  } else if (fv) {
     radices = fv->radices;
   } else {
     bool ok = true;
@@ -472,7 +476,7 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   st = get_twiddles(p, radices, &tt);
   if (st) return st;
   a.tw = tt->d;
-  a.n = fv ? fv->n : (bt ? bt->M : g.n);
+  a.n = fv && !fv->mixed ? fv->n : (bt ? bt->M : g.n);
   if (bt) {
     a.blue = 1;
     a.nblue = g.n;
@@ -485,11 +489,13 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   a.C0 = (g.io == IO_C2C || (fv && fv->io == IO_DTT4)) ? g.C0r : (g.C0r + 1) / 2;
   a.C1 = g.C1;
   if (fv) {
-    s.TX = fv->TX;
-    s.nthreads = fv->NT;
-    s.lds_bytes = fv->lds_bytes;
-    s.ldj = fv->ldj;
-    s.ldt = fv->ldt;
+    if (!fv->mixed) {
+      s.TX = fv->TX;
+      s.nthreads = fv->NT;
+      s.lds_bytes = fv->lds_bytes;
+      s.ldj = fv->ldj;
+      s.ldt = fv->ldt;
+    }
     st = hip_check(fv->prepare(), "hipFuncSetAttribute(fast kernel)");
     if (st) return st;
   } else {
@@ -509,6 +515,9 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   a.out_sj = g.out_sj;
   a.ldj = s.ldj;
   a.ldt = s.ldt;
+  a.rows = s.rows;
+  a.nthreads = s.nthreads;
+  a.lds_bytes = (int)s.lds_bytes;
   a.nh = g.n / 2 + 1;
   a.dtt = g.dtt;
   a.dtt_first = g.dtt_first;
@@ -549,6 +558,12 @@ int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, 
             v.n == g.n)
           g.cands.push_back(&v);
     }
+    // then the kernels of any length (not beside the matrix-core ones: a
+    // split plan keeps those); the default where no tile is compiled for it
+    if (g.cands.empty() || !g.cands[0]->mf)
+      for (const FastVariant &v : fast_registry())
+        if (v.mixed && v.rb == p->rb && v.io == io && v.lines == (axis == 0 ? 1 : 0) && mixed_runs(v, g.n))
+          g.cands.push_back(&v);
   }
   return configure(p, idx, g.cands.empty() ? -1 : 0);
 }
@@ -2273,7 +2288,9 @@ int run_stage_packed(d2dhip_plan_s *p, int stage, const void *in, void *out, int
   // the specialised kernel's fused form, if it has one
   const int io = packj == 1 ? IO_YPK : packj == 2 ? IO_YUN : IO_YUP;
   const FastVariant *v = p->fast[stage], *twin = nullptr;
-  if (v) {
+  if (v && v->mixed) {
+    twin = v;  // (applies the tables itself)
+  } else if (v) {
     std::string want = v->name;
     const size_t at = want.find(" c2c");
     if (at != std::string::npos) {
@@ -2931,7 +2948,7 @@ int d2dhip_batch_launch(d2dhip_batch b) {
     for (const auto &pp : b->parts)
       for (const auto &q : pp) {
         const MultiGroup *g = b->d_multi + q.m0;
-        const int st = q.fv ? q.fv->launch_multi(g, q.ng, q.tiles, b->stream)
+        const int st = q.fv ? q.fv->launch_multi(g, q.ng, q.tiles, q.nthreads, q.lds, b->stream)
                             : launch_general_multi(b->rb, g, q.ng, q.tiles, q.nthreads, q.lds,
                                                    b->stream);
         if (st) return st;
