@@ -47,9 +47,12 @@ const std::vector<PersistKind> &persist_kinds(int rb);
 int batch_fast_prepare(int rb, size_t lds, int *blocks_per_cu);
 int launch_batch_fast(int rb, const BatchQueue &q, int blocks, size_t lds, hipStream_t st);
 // The kernels of any length (mixed_impl.h); whether one of them runs length
-// n; and the tile and radix schedule that it takes (C0 tile-level columns).
+// n, the length of its transform (longer than n for Bluestein's algorithm,
+// mixed = 3), and the tile and radix schedule that it takes (C0 tile-level
+// columns).
 std::vector<FastVariant> mixed_variants();
 bool mixed_runs(const FastVariant &v, int n);
+int mixed_length(const FastVariant &v, int n);
 bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &radices, AxisShape &s);
 // The split-BF16 matrix-core variants (mfma_kernels.hip).
 std::vector<FastVariant> mf_variants();

@@ -21,7 +21,15 @@
 //   n = 100  2.0 / 2.7 / 2.3 -> 5.2 / 5.5 / 5.1
 //   n = 405  1.9 / 3.0 / 2.4 -> 4.4 / 4.7 / 4.6
 //   n = 1000 1.3 / 2.0 / 1.6 -> 3.9 / 4.9 / 4.9
-// What bounds it: up to 600 points the HBM rate of the access pattern; longer
+// Class 2 ("chirp") runs lengths with a prime factor above 17 by Bluestein's
+// algorithm over a smooth length m >= 2n - 1, in place (the general kernel
+// pads to a power of two and sweeps the LDS tile twelve times at n = 382):
+// columns of 107 / 191 / 382 / 1021 points 1.0 / 0.8 / 0.8 / 0.9 -> 1.9 / 2.1 /
+// 1.9 / 1.7 TB/s.  It is bound by latency and the texture path: at n = 382 the
+// vector units are busy 40 % of the time, the twiddle, chirp and spectrum
+// loads keep the address unit busy half of it.  Radices end at 12, where
+// FP64 still fits 128 VGPRs with a pass's twiddles loaded ahead.
+// What bounds the Stockham classes: up to 600 points the HBM rate of the access pattern; longer
 // columns the workgroups per CU, since a tile of 8 columns takes over half
 // of the LDS.
 #pragma once
@@ -41,7 +49,7 @@ namespace {
 constexpr int mx_nb(int r) { return r > 5 ? 1 : (10 / r < 4 ? 10 / r : 4); }
 
 // Radices by kernel class: 0 the codelets that fit 128 VGPRs in FP64 at 1024
-// threads, 1 the large primes too (512 threads).
+// threads, 1 the large primes too (512 threads), 2 (chirp) those of 0.
 template <int CLS, class F>
 __device__ __forceinline__ void radix_case(int r, F &&f) {
   switch (r) {
@@ -55,9 +63,11 @@ __device__ __forceinline__ void radix_case(int r, F &&f) {
     case 9: f(std::integral_constant<int, 9>{}); break;
     case 10: f(std::integral_constant<int, 10>{}); break;
     case 12: f(std::integral_constant<int, 12>{}); break;
-    case 15: f(std::integral_constant<int, 15>{}); break;
-    case 16: f(std::integral_constant<int, 16>{}); break;
     default:
+      if constexpr (CLS != 2) {
+        if (r == 15) f(std::integral_constant<int, 15>{});
+        else if (r == 16) f(std::integral_constant<int, 16>{});
+      }
       if constexpr (CLS == 1) {
         if (r == 11) f(std::integral_constant<int, 11>{});
         else if (r == 13) f(std::integral_constant<int, 13>{});
@@ -85,7 +95,9 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   extern __shared__ __align__(16) unsigned char lds_raw[];
   cpx<T> *lds = reinterpret_cast<cpx<T> *>(lds_raw);
   constexpr bool PAIRED = IO == IO_R2C || IO == IO_C2R;
-  const int n = d->n, TX = d->TX, lg = d->log2TX, rows = d->rows, np = d->npass;
+  constexpr bool CHIRP = CLS == 2;
+  // n: points of a line; m: points of the transform
+  const int m = d->n, n = CHIRP ? d->nblue : m, TX = d->TX, lg = d->log2TX, rows = d->rows, np = d->npass;
   const int tid = threadIdx.x, nthr = blockDim.x;
   const long long tiles0 = d->tiles0;
   const long long c1 = tile / tiles0;
@@ -107,7 +119,6 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
                             (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->in_b0 : 0);
   const long long out_base = (IO == IO_C2R ? ca : c0) * d->out_s0 + c1 * d->out_s1 +
                              (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->out_b0 : 0);
-  const void *tw = d->tw;
   // LDS: [point][column] for strided columns; [line][point] with one pad
   // point in 17 for contiguous lines, whose first exchange writes with the
   // stride of the first radix
@@ -120,7 +131,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   // values of the first pass (and whole transforms of one pass) from HBM
   auto load = [&](auto rc, auto &v) __attribute__((always_inline)) {
     constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-    const int nb = n / R;
+    const int nb = m / R;
     const long long step = (long long)nb * sji;
     if constexpr (IO == IO_R2C) {
       // adjacent columns whose pairs are aligned: one load per pair
@@ -133,10 +144,12 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
           const long long o = in_base + (long long)b * sji;
           if (vec && two) {
 #pragma unroll
-            for (int s = 0; s < R; ++s) v[q * R + s] = gload<T>(in, (o + s * step) >> 1);
+            for (int s = 0; s < R; ++s)
+              if (!CHIRP || b + s * nb < n) v[q * R + s] = gload<T>(in, (o + s * step) >> 1);
           } else {
 #pragma unroll
             for (int s = 0; s < R; ++s) {
+              if (CHIRP && b + s * nb >= n) continue;
               v[q * R + s].x = gload_r<T>(in, o + s * step);
               v[q * R + s].y = two ? gload_r<T>(in, o + s * step + d->in_s0) : T(0);
             }
@@ -154,14 +167,16 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
             for (int s0 = 0; s0 < R; s0 += 4) {  // four table reads, then their loads
               long long off[4];
 #pragma unroll
-              for (int s = s0; s < R && s < s0 + 4; ++s) off[s - s0] = packj_offset(d, b + s * nb, c1);
+              for (int s = s0; s < R && s < s0 + 4; ++s)
+                if (!CHIRP || b + s * nb < n) off[s - s0] = packj_offset(d, b + s * nb, c1);
 #pragma unroll
               for (int s = s0; s < R && s < s0 + 4; ++s)
-                v[q * R + s] = gload<T>(in, o + s * step + off[s - s0]);
+                if (!CHIRP || b + s * nb < n) v[q * R + s] = gload<T>(in, o + s * step + off[s - s0]);
             }
           } else {
 #pragma unroll
-            for (int s = 0; s < R; ++s) v[q * R + s] = gload<T>(in, o + s * step);
+            for (int s = 0; s < R; ++s)
+              if (!CHIRP || b + s * nb < n) v[q * R + s] = gload<T>(in, o + s * step);
           }
           if (conj) {
 #pragma unroll
@@ -174,7 +189,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   // outputs j = b + s * (n / R) of the last pass to HBM
   auto store = [&](auto rc, auto &v) __attribute__((always_inline)) {
     constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-    const int nb = n / R;
+    const int nb = m / R;
     const long long step = (long long)nb * sjo;
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -184,6 +199,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
         if constexpr (IO == IO_C2R) {  // the pre-phase stored conj(Z): z = conj(result)
 #pragma unroll
           for (int s = 0; s < R; ++s) {
+            if (CHIRP && b + s * nb >= n) continue;
             gstore_r<T>(out, o + s * step, v[q * R + s].x);
             if (two) gstore_r<T>(out, o + s * step + d->out_s0, -v[q * R + s].y);
           }
@@ -198,14 +214,16 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
             for (int s0 = 0; s0 < R; s0 += 4) {
               long long off[4];
 #pragma unroll
-              for (int s = s0; s < R && s < s0 + 4; ++s) off[s - s0] = packj_offset_in(tab, b + s * nb, c1);
+              for (int s = s0; s < R && s < s0 + 4; ++s)
+                if (!CHIRP || b + s * nb < n) off[s - s0] = packj_offset_in(tab, b + s * nb, c1);
 #pragma unroll
               for (int s = s0; s < R && s < s0 + 4; ++s)
-                gstore<T>(out, o + s * step + off[s - s0], v[q * R + s]);
+                if (!CHIRP || b + s * nb < n) gstore<T>(out, o + s * step + off[s - s0], v[q * R + s]);
             }
           } else {
 #pragma unroll
-            for (int s = 0; s < R; ++s) gstore<T>(out, o + s * step, v[q * R + s]);
+            for (int s = 0; s < R; ++s)
+              if (!CHIRP || b + s * nb < n) gstore<T>(out, o + s * step, v[q * R + s]);
           }
         }
       }
@@ -274,94 +292,231 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 
   // ---- passes --------------------------------------------------------------------
   constexpr bool HBM_IN = IO != IO_C2R, HBM_OUT = IO != IO_R2C;
-  if (HBM_IN && HBM_OUT && np == 1) {
-    radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
-      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-      cpx<T> v[NB * R];
-      load(rc, v);
-      if (row < rows) dft<T, R>(v);  // n == R: one butterfly per column
-      store(rc, v);
-    });
-    return;
+  if constexpr (HBM_IN && HBM_OUT && !CHIRP) {
+    if (np == 1) {
+      radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+        cpx<T> v[NB * R];
+        load(rc, v);
+        if (row < rows) dft<T, R>(v);  // n == R: one butterfly per column
+        store(rc, v);
+      });
+      return;
+    }
   }
-  int p = 0;
-  if constexpr (HBM_IN) {
-    radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
-      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-      const int nb = n / R;
-      cpx<T> v[NB * R];
-      load(rc, v);
-#pragma unroll
-      for (int q = 0; q < NB; ++q) {
-        const int b = row + q * rows;
-        if (b < nb) {
-          dft<T, R>(&v[q * R]);
-#pragma unroll
-          for (int s = 0; s < R; ++s) lds[A(b * R + s, t)] = v[q * R + s];
-        }
-      }
-    });
-    __syncthreads();
-    p = 1;
-  }
-  const int pmid = HBM_OUT ? np - 1 : np;
-  for (; p < pmid; ++p) {
-    const int L = d->pass[p].L, tw_off = d->pass[p].tw_off;
-    const float invL = d->pass[p].invL;
-    // a zero the compiler cannot see through: it would otherwise hoist the
-    // loop-invariant address parts of every radix's case out of the loop, far
-    // more than there are registers (430 bytes of spill per lane)
-    int zero;
-    asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
-    const int n_ = n + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
-    radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
-      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-      const int nb = n_ / R;
-      cpx<T> v[NB * R];
-      lds_read(rc, v, nb, row_, rows_, t_);
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < NB; ++q) {
-        const int b = row_ + q * rows_;
-        if (b < nb) {
-          int g, k;
-          est_divmod(b, L, invL, g, k);
-          if (L > 1) {
-#pragma unroll
-            for (int s = 1; s < R; ++s)
-              v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + k * (R - 1) + (s - 1)));
-          }
-          dft<T, R>(&v[q * R]);
-          const int jb = g * L * R + k;
-#pragma unroll
-          for (int s = 0; s < R; ++s) lds[A(jb + s * L, t_)] = v[q * R + s];
-        }
-      }
-    });
-    __syncthreads();
-  }
-  if constexpr (HBM_OUT) {
-    const int tw_off = d->pass[np - 1].tw_off;
+  const void *tw = d->tw;
+  if constexpr (CHIRP) {
+    // y_k = c_k sum_j (x_j c_j) w_{k-j}: the first transform runs its passes
+    // from the last to the first by decimation in frequency, the inverse one
+    // (as conj(DFT(conj(.)))) from the first to the last by decimation in time,
+    // all in place: a lane writes a butterfly back to the points it read.  So
+    // an exchange takes one barrier, both transforms share one twiddle table,
+    // and the spectrum stays in the first one's order (bhat is stored in it).
+    // The twiddles of a pass are loaded before its points.
+    const T invm = T(1) / (T)m;
+    const int tw_last = d->pass[np - 1].tw_off;
     radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
       constexpr int R = decltype(rc)::value, NB = mx_nb(R);
-      const int nb = n / R;  // = L: every butterfly of the last pass is its own k
+      const int nb = m / R;
       cpx<T> v[NB * R];
-      lds_read(rc, v, nb, row, rows, t);
+#pragma unroll
+      for (int i = 0; i < NB * R; ++i) v[i] = cpx<T>{T(0), T(0)};
+      if constexpr (HBM_IN) {
+        load(rc, v);
+      } else {  // the merged spectra, already in LDS
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          const int b = row + q * rows;
+#pragma unroll
+          for (int s = 0; s < R; ++s)
+            if (b < nb && b + s * nb < n) v[q * R + s] = lds[A(b + s * nb, t)];
+        }
+      }
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         const int b = row + q * rows;
         if (b < nb) {
-          if (nb > 1) {
 #pragma unroll
-            for (int s = 1; s < R; ++s)
-              v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + b * (R - 1) + (s - 1)));
-          }
+          for (int s = 0; s < R; ++s)
+            if (b + s * nb < n) v[q * R + s] = cmul(v[q * R + s], gload<T>(d->chirp, b + s * nb));
           dft<T, R>(&v[q * R]);
+          lds[A(b, t)] = v[q * R];
+#pragma unroll
+          for (int s = 1; s < R; ++s)
+            lds[A(b + s * nb, t)] = cmul(v[q * R + s], gload<T>(tw, tw_last + b * (R - 1) + (s - 1)));
         }
       }
-      store(rc, v);
     });
+    __syncthreads();
+    for (int w = 0; w < 2 * np - 3; ++w) {
+      // w < np - 2: passes np - 2 .. 1 of the first transform; w = np - 2:
+      // pass 0 of both; then passes 1 .. np - 2 of the second
+      const int turn = np - 2, p = w < turn ? turn - w : w - turn;
+      const int L = d->pass[p].L, tw_off = d->pass[p].tw_off;
+      const float invL = d->pass[p].invL;
+      // a zero the compiler cannot see through: it would otherwise hoist the
+      // loop-invariant address parts of every radix's case out of the loop,
+      // far more than there are registers
+      int zero;
+      asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+      const int m_ = m + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
+      radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+        const int nb = m_ / R;
+        if (w == turn) {
+#pragma unroll
+          for (int q = 0; q < NB; ++q) {
+            const int b = row_ + q * rows_;
+            if (b < nb) {
+              cpx<T> v[R], f[R];
+#pragma unroll
+              for (int s = 0; s < R; ++s) f[s] = gload<T>(d->bhat, b * R + s);
+#pragma unroll
+              for (int s = 0; s < R; ++s) v[s] = lds[A(b * R + s, t_)];
+              dft<T, R>(v);
+#pragma unroll
+              for (int s = 0; s < R; ++s) v[s] = cconj(cmul(v[s], f[s]));
+              dft<T, R>(v);
+#pragma unroll
+              for (int s = 0; s < R; ++s) lds[A(b * R + s, t_)] = v[s];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < NB; ++q) {
+            const int b = row_ + q * rows_;
+            if (b < nb) {
+              int g, k;
+              est_divmod(b, L, invL, g, k);
+              const int jb = g * L * R + k;
+              cpx<T> v[R], f[R];
+#pragma unroll
+              for (int s = 1; s < R; ++s) f[s] = gload<T>(tw, tw_off + k * (R - 1) + (s - 1));
+#pragma unroll
+              for (int s = 0; s < R; ++s) v[s] = lds[A(jb + s * L, t_)];
+              if (w > turn) {
+#pragma unroll
+                for (int s = 1; s < R; ++s) v[s] = cmul(v[s], f[s]);
+              }
+              dft<T, R>(v);
+              if (w < turn) {
+#pragma unroll
+                for (int s = 1; s < R; ++s) v[s] = cmul(v[s], f[s]);
+              }
+#pragma unroll
+              for (int s = 0; s < R; ++s) lds[A(jb + s * L, t_)] = v[s];
+            }
+          }
+        }
+      });
+      __syncthreads();
+    }
+    radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      const int nb = m / R;
+      cpx<T> v[NB * R];
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          cpx<T> f[R];
+#pragma unroll
+          for (int s = 1; s < R; ++s) f[s] = gload<T>(tw, tw_last + b * (R - 1) + (s - 1));
+          v[q * R] = lds[A(b, t)];
+#pragma unroll
+          for (int s = 1; s < R; ++s) v[q * R + s] = cmul(lds[A(b + s * nb, t)], f[s]);
+          dft<T, R>(&v[q * R]);
+#pragma unroll
+          for (int s = 0; s < R; ++s)
+            if (b + s * nb < n) {
+              const cpx<T> y = cmul(cconj(v[q * R + s]), gload<T>(d->chirp, b + s * nb));
+              v[q * R + s] = cpx<T>{y.x * invm, y.y * invm};
+              if constexpr (!HBM_OUT) lds[A(b + s * nb, t)] = v[q * R + s];
+            }
+        }
+      }
+      if constexpr (HBM_OUT) store(rc, v);
+    });
+    if constexpr (!HBM_OUT) __syncthreads();
   } else {
+    int p = 0;
+    if constexpr (HBM_IN) {
+      radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+        const int nb = n / R;
+        cpx<T> v[NB * R];
+        load(rc, v);
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          const int b = row + q * rows;
+          if (b < nb) {
+            dft<T, R>(&v[q * R]);
+#pragma unroll
+            for (int s = 0; s < R; ++s) lds[A(b * R + s, t)] = v[q * R + s];
+          }
+        }
+      });
+      __syncthreads();
+      p = 1;
+    }
+    const int pmid = HBM_OUT ? np - 1 : np;
+    for (; p < pmid; ++p) {
+      const int L = d->pass[p].L, tw_off = d->pass[p].tw_off;
+      const float invL = d->pass[p].invL;
+      // (an opaque zero, as above: 430 bytes of spill per lane without it)
+      int zero;
+      asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
+      const int n_ = n + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
+      radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+        const int nb = n_ / R;
+        cpx<T> v[NB * R];
+        lds_read(rc, v, nb, row_, rows_, t_);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          const int b = row_ + q * rows_;
+          if (b < nb) {
+            int g, k;
+            est_divmod(b, L, invL, g, k);
+            if (L > 1) {
+#pragma unroll
+              for (int s = 1; s < R; ++s)
+                v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + k * (R - 1) + (s - 1)));
+            }
+            dft<T, R>(&v[q * R]);
+            const int jb = g * L * R + k;
+#pragma unroll
+            for (int s = 0; s < R; ++s) lds[A(jb + s * L, t_)] = v[q * R + s];
+          }
+        }
+      });
+      __syncthreads();
+    }
+    if constexpr (HBM_OUT) {
+      const int tw_off = d->pass[np - 1].tw_off;
+      radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+        const int nb = n / R;  // = L: every butterfly of the last pass is its own k
+        cpx<T> v[NB * R];
+        lds_read(rc, v, nb, row, rows, t);
+#pragma unroll
+        for (int q = 0; q < NB; ++q) {
+          const int b = row + q * rows;
+          if (b < nb) {
+            if (nb > 1) {
+#pragma unroll
+              for (int s = 1; s < R; ++s)
+                v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + b * (R - 1) + (s - 1)));
+            }
+            dft<T, R>(&v[q * R]);
+          }
+        }
+        store(rc, v);
+      });
+    }
+  }
+  if constexpr (!HBM_OUT) {
     // A[k] = (Z[k] + conj Z[n-k]) / 2 and B[k] = (Z[k] - conj Z[n-k]) / (2i)
     const T half = T(0.5);
     const int total = TX * nh;
@@ -391,10 +546,10 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 
 // Threads a workgroup may have, and the waves per SIMD its registers leave
 // room for.
-constexpr int mx_threads(int cls) { return cls == 0 ? 1024 : 512; }
+constexpr int mx_threads(int cls) { return cls == 1 ? 512 : 1024; }
 template <typename T>
 constexpr int mx_wpe(int cls) {
-  return cls == 0 ? (sizeof(T) == 8 ? 4 : 6) : (sizeof(T) == 8 ? 2 : 4);
+  return cls != 1 ? (sizeof(T) == 8 ? 4 : 6) : (sizeof(T) == 8 ? 2 : 4);
 }
 
 // One grid (ng = 0: the stage of the arguments), or the tiles of several
@@ -473,14 +628,14 @@ FastVariant mixed_variant(const char *name) {
   return v;
 }
 
-// c2c, r2c and c2r, strided columns and contiguous lines, both classes
-#define D2D_MIXED(T, IO, LINES, TAG)                               \
-  mixed_variant<T, IO, LINES, 0>(#T " mixed " TAG),                \
-      mixed_variant<T, IO, LINES, 1>(#T " mixed " TAG " primes")
-#define D2D_MIXED_ALL(T)                                                   \
-  D2D_MIXED(T, IO_C2C, false, "c2c"), D2D_MIXED(T, IO_C2C, true, "c2c"),   \
-  D2D_MIXED(T, IO_R2C, false, "r2c"), D2D_MIXED(T, IO_R2C, true, "r2c"),   \
-  D2D_MIXED(T, IO_C2R, false, "c2r"), D2D_MIXED(T, IO_C2R, true, "c2r")
+// c2c, r2c and c2r of one class, strided columns and contiguous lines
+#define D2D_MIXED_ALL(T, CLS, TAG)                                            \
+  mixed_variant<T, IO_C2C, false, CLS>(#T " mixed c2c" TAG),                  \
+      mixed_variant<T, IO_C2C, true, CLS>(#T " mixed c2c" TAG),               \
+      mixed_variant<T, IO_R2C, false, CLS>(#T " mixed r2c" TAG),              \
+      mixed_variant<T, IO_R2C, true, CLS>(#T " mixed r2c" TAG),               \
+      mixed_variant<T, IO_C2R, false, CLS>(#T " mixed c2r" TAG),              \
+      mixed_variant<T, IO_C2R, true, CLS>(#T " mixed c2r" TAG)
 
 }  // namespace
 

@@ -1,0 +1,144 @@
+// mixed_plan.cpp -- the tile and radix schedule that a kernel of any length
+// (mixed_impl.h) takes for a length, and the list of those kernels.
+#include <algorithm>
+
+#include "mixed_impl.h"
+
+namespace d2dhip {
+
+namespace {
+
+constexpr int kRadices[3][15] = {{16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2},
+                                 {17, 16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2},
+                                 {12, 10, 9, 8, 7, 6, 5, 4, 3, 2}};
+
+// Least rows per column of a schedule (every pass within its butterflies per
+// lane), and the work of its passes in lanes, idle ones counted.
+int least_rows(int n, const std::vector<int> &r) {
+  int rows = 1;
+  for (int x : r) rows = std::max(rows, (n / x + mx_nb(x) - 1) / mx_nb(x));
+  return rows;
+}
+double sched_cost(int n, int rows, const std::vector<int> &r) {
+  double c = 0;
+  for (int x : r) c += (double)rows * ((n / x + rows - 1) / rows) * x / n;
+  return c + (double)r.size();
+}
+
+// Schedules of n over non-increasing radices, at most 5 passes; keeps the
+// cheapest.
+void search(int n, int left, int from, int cls, std::vector<int> &cur, std::vector<int> &best, int &rows,
+            double &cost) {
+  if (left == 1) {
+    // the least rows, or up to half as many again where they divide a pass evenly
+    const int r0 = least_rows(n, cur);
+    auto take = [&](int r) {
+      if (r < r0 || r > r0 + r0 / 2) return;
+      const double c = sched_cost(n, r, cur);
+      if (c < cost - 1e-9 || (c < cost + 1e-9 && best == cur && r < rows)) {
+        cost = c;
+        best = cur;
+        rows = r;
+      }
+    };
+    take(r0);
+    for (int x : cur)
+      for (int q = 1; q <= 4; ++q) take((n / x + q - 1) / q);
+    return;
+  }
+  if (cur.size() == 5) return;
+  for (int i = from; i < 15 && kRadices[cls][i]; ++i) {
+    const int x = kRadices[cls][i];
+    if (left % x) continue;
+    cur.push_back(x);
+    search(n, left / x, i, cls, cur, best, rows, cost);
+    cur.pop_back();
+  }
+}
+
+}  // namespace
+
+// A class takes the lengths that the lighter one does not, up to six points
+// per thread of a block (the fewest a lane may have in a pass) and one
+// column per tile.
+bool mixed_runs(const FastVariant &v, int n) {
+  const int cls = v.mixed - 1;
+  int left = n;
+  for (int x : {2, 3, 5, 7}) while (left > 0 && left % x == 0) left /= x;
+  const bool smooth = left == 1;
+  for (int x : {11, 13, 17}) while (left > 0 && left % x == 0) left /= x;
+  if (n < 2 || cls != (smooth ? 0 : left == 1 ? 1 : 2)) return false;
+  const int m = mixed_length(v, n);
+  return m <= 6 * mx_threads(cls) && (size_t)m * 17 / 16 * 2 * v.rb + 64 <= (size_t)kMaxLds;
+}
+
+// Length of the transform: n itself, or for a chirp the least m >= 2n - 1
+// among 2^k times 1, 3, 5, 9 and 15 (m = 768 runs n = 382 at 1.8 TB/s, 800
+// to 960 at 1.6 to 1.7, 1024 at 1.5).
+int mixed_length(const FastVariant &v, int n) {
+  if (v.mixed != 3) return n;
+  int best = 0;
+  for (int f : {1, 3, 5, 9, 15}) {
+    int m = f;
+    while (m < 2 * n - 1) m *= 2;
+    if (!best || m < best) best = m;
+  }
+  return best;
+}
+
+// Columns: the widest rows (256 bytes at most) that leave room for two
+// workgroups on a CU, and more columns while the block stays below 256
+// threads and 40 KB.  FP64 columns, 16 / 8 / 4 wide, TB/s: 270 points 5.0 /
+// 4.7 / 4.7, 512 points 4.7 / 4.7 / 4.2, 720 points 3.7 / 3.7 / 3.9, 1024
+// points 3.7 / 3.8 / 4.1.  Lines: as many as make 256 threads (64 to 512
+// threads lie within 5 %).
+bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &radices, AxisShape &s) {
+  const int cls = v.mixed - 1, cb = 2 * v.rb;
+  if (!mixed_runs(v, n)) return false;
+  n = mixed_length(v, n);
+  std::vector<int> cur;
+  double cost = 1e30;
+  int rows = 0;
+  search(n, n, 0, cls, cur, radices, rows, cost);
+  if (!rows) return false;
+  if (v.lines)  // an odd first radix: its stride spreads the first exchange over the banks
+    std::stable_partition(radices.begin(), radices.end(), [](int x) { return x % 2 == 1; });
+  const int ldt = v.lines ? ((n - 1) + ((n - 1) >> 4) + 1) | 1 : n;
+  const int maxt = mx_threads(cls);
+  auto lds = [&](int tx) { return (size_t)tx * ldt * cb; };
+  int tx = v.lines ? 1 : (cls == 2 ? 128 : 256) / cb;
+  while (tx > 1 && (tx * rows > maxt || lds(tx) > (size_t)kMaxLds / 2)) tx >>= 1;
+  if (tx * rows > maxt || lds(tx) > (size_t)kMaxLds) return false;
+  while (tx < C0 && tx < 64 && 2 * tx * rows <= 256 && lds(2 * tx) <= 40 * 1024) tx *= 2;
+  // chirps wait on their barriers: blocks of a multiple of four waves load the
+  // four SIMDs alike (m = 768, 4 columns: 1.96 TB/s with 512 threads, 1.85
+  // with 384)
+  if (cls == 2 && tx * rows > 256)
+    while (tx * rows % 256 && tx * (rows + 1) <= maxt) ++rows;
+  s.TX = tx;
+  s.rows = rows;
+  s.nthreads = (tx * rows + 63) / 64 * 64;
+  s.lds_bytes = lds(tx);
+  s.ldj = v.lines ? 1 : tx;
+  s.ldt = v.lines ? ldt : 1;
+  return true;
+}
+
+// compiled in mixed_f64.hip, mixed_f64_chirp.hip, mixed_f32.hip and
+// mixed_f32_chirp.hip
+std::vector<FastVariant> mixed_variants_f64();
+std::vector<FastVariant> mixed_variants_f64_chirp();
+std::vector<FastVariant> mixed_variants_f32();
+std::vector<FastVariant> mixed_variants_f32_chirp();
+
+std::vector<FastVariant> mixed_variants() {
+  std::vector<FastVariant> v;
+  for (auto part : {mixed_variants_f64, mixed_variants_f64_chirp, mixed_variants_f32,
+                    mixed_variants_f32_chirp}) {
+    const std::vector<FastVariant> q = part();
+    v.insert(v.end(), q.begin(), q.end());
+  }
+  return v;
+}
+
+}  // namespace d2dhip

@@ -65,7 +65,7 @@ struct d2dhip_plan_s {
   unsigned flags = 0;
   hipStream_t stream = nullptr;
   std::map<std::vector<int>, TwTable> tw;
-  std::map<int, BlueTables> blue;
+  std::map<std::vector<int>, BlueTables> blue;  // by line length, convolution length, spectrum order
   std::map<int, void *> dtw;  // DCT / DST twiddle tables by length
   // Stage descriptors: 0-2 c2c along x, y, z of the (nx,ny,nz) pencil;
   // 3 the real-to-complex stage; 4 the spectral y stage; 5 the other
@@ -365,55 +365,97 @@ StageIo cols_view(int axis, long long n1, long long n2, long long n3) {
   return v;
 }
 
-// Bluestein tables of line length n: c_j = exp(-i pi j^2/n) (j < n) and the
-// length-M DFT of w_m = exp(+i pi m^2/n) wrapped as w[m] = w[M-m] = w_m,
-// evaluated in long double with j^2 reduced mod 2n exactly.
-int get_bluestein(d2dhip_plan_s *p, int n, const BlueTables **out) {
-  auto it = p->blue.find(n);
+// DFT (sign -1) of the n points of w, st apart, into out, in long double: by
+// the least prime factor r, the r sub-transforms then combined in place.
+// root[i] = exp(-2 pi i / M), M the whole transform's length (a multiple of n).
+struct LdCpx {
+  long double re = 0, im = 0;
+};
+LdCpx ld_mul(LdCpx a, LdCpx b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
+void host_dft(const LdCpx *w, long long st, int n, LdCpx *out, const LdCpx *root, int M) {
+  if (n == 1) {
+    out[0] = w[0];
+    return;
+  }
+  int r = 2;
+  while (r * r <= n && n % r) ++r;
+  if (n % r) r = n;
+  const int m = n / r, step = M / n;
+  for (int q = 0; q < r; ++q) host_dft(w + q * st, st * r, m, out + (size_t)q * m, root, M);
+  if (r == 2) {
+    for (int k = 0; k < m; ++k) {
+      const LdCpx a = out[k], b = k ? ld_mul(out[m + k], root[(long long)k * step]) : out[m];
+      out[k] = {a.re + b.re, a.im + b.im};
+      out[m + k] = {a.re - b.re, a.im - b.im};
+    }
+    return;
+  }
+  std::vector<LdCpx> t(r);
+  for (int k = 0; k < m; ++k) {
+    for (int q = 0; q < r; ++q) t[q] = ld_mul(out[(size_t)q * m + k], root[(long long)q * k * step]);
+    for (int j = 0; j < r; ++j) {
+      LdCpx a = t[0];
+      for (int q = 1; q < r; ++q) {
+        const LdCpx v = ld_mul(t[q], root[(long long)q * j % r * m * step]);
+        a.re += v.re;
+        a.im += v.im;
+      }
+      out[(size_t)j * m + k] = a;
+    }
+  }
+}
+
+// Bluestein tables of line length n over convolution length M: c_j =
+// exp(-i pi j^2/n) (j < n) and the length-M DFT of w_m = exp(+i pi m^2/n)
+// wrapped as w[m] = w[M-m] = w_m, evaluated in long double with j^2 reduced
+// mod 2n exactly.  `order`: the radices of a schedule whose transform leaves
+// the spectrum in its in-place order, in which bhat is then stored (position
+// d0 + r0 (d1 + r1 (d2 + ...)) holds frequency d0 M/r0 + d1 M/(r0 r1) + ...);
+// empty: natural order.
+int get_bluestein(d2dhip_plan_s *p, int n, int M, const std::vector<int> &order, const BlueTables **out) {
+  std::vector<int> key = {n, M};
+  key.insert(key.end(), order.begin(), order.end());
+  auto it = p->blue.find(key);
   if (it != p->blue.end()) {
     *out = &it->second;
     return D2DHIP_SUCCESS;
   }
   BlueTables b;
-  b.M = 1;
-  while (b.M < 2 * n - 1) b.M *= 2;
-  const int M = b.M;
-  std::vector<long double> cr(n), ci(n), wr(M, 0.0L), wi(M, 0.0L);
+  b.M = M;
+  std::vector<long double> cr(n), ci(n);
+  std::vector<LdCpx> w0(M), w(M), root(M);
   for (int j = 0; j < n; ++j) {
     long double c, s;
     unit_root(((long long)j * j) % (2LL * n), 2LL * n, c, s);
     cr[j] = c;
     ci[j] = -s;
-    wr[j] = c;
-    wi[j] = s;
-    if (j > 0) {
-      wr[M - j] = c;
-      wi[M - j] = s;
-    }
+    w0[j] = {c, s};
+    if (j > 0) w0[M - j] = {c, s};
   }
-  // iterative radix-2 DFT of w (sign -1), bit-reversed input order
-  for (int i = 1, j = 0; i < M; ++i) {
-    int bit = M >> 1;
-    for (; j & bit; bit >>= 1) j ^= bit;
-    j ^= bit;
-    if (i < j) {
-      std::swap(wr[i], wr[j]);
-      std::swap(wi[i], wi[j]);
+  // exp(-2 pi i k / M): an octant, reflected (any M that is no multiple of 8
+  // is at most 60)
+  for (int k = 0; k < M; ++k) {
+    if (M % 8 == 0 && 8 * k > M) {
+      const LdCpx a = root[4 * k <= M ? M / 4 - k : 2 * k <= M ? M / 2 - k : M - k];
+      if (4 * k <= M) root[k] = {-a.im, -a.re};
+      else if (2 * k <= M) root[k] = {-a.re, a.im};
+      else root[k] = {a.re, -a.im};
+      continue;
     }
+    unit_root(k, M, root[k].re, root[k].im);
+    root[k].im = -root[k].im;
   }
-  for (int len = 2; len <= M; len <<= 1) {
-    for (int k = 0; k < len / 2; ++k) {
-      long double c, s;
-      unit_root(k, len, c, s);
-      const long double tr = c, ti = -s;
-      for (int i = k; i < M; i += len) {
-        const int j = i + len / 2;
-        const long double xr = wr[j] * tr - wi[j] * ti, xi = wr[j] * ti + wi[j] * tr;
-        wr[j] = wr[i] - xr;
-        wi[j] = wi[i] - xi;
-        wr[i] += xr;
-        wi[i] += xi;
+  host_dft(w0.data(), 1, M, w.data(), root.data(), M);
+  if (!order.empty()) {
+    const std::vector<LdCpx> nat = w;
+    for (int pos = 0; pos < M; ++pos) {
+      int q = pos, f = 0, step = M;
+      for (int r : order) {
+        step /= r;
+        f += q % r * step;
+        q /= r;
       }
+      w[pos] = nat[f];
     }
   }
   const int rb = p->rb;
@@ -429,18 +471,18 @@ int get_bluestein(d2dhip_plan_s *p, int n, const BlueTables **out) {
   }
   for (int m = 0; m < M; ++m) {
     if (rb == 8) {
-      reinterpret_cast<double *>(hw.data())[2 * m] = (double)wr[m];
-      reinterpret_cast<double *>(hw.data())[2 * m + 1] = (double)wi[m];
+      reinterpret_cast<double *>(hw.data())[2 * m] = (double)w[m].re;
+      reinterpret_cast<double *>(hw.data())[2 * m + 1] = (double)w[m].im;
     } else {
-      reinterpret_cast<float *>(hw.data())[2 * m] = (float)wr[m];
-      reinterpret_cast<float *>(hw.data())[2 * m + 1] = (float)wi[m];
+      reinterpret_cast<float *>(hw.data())[2 * m] = (float)w[m].re;
+      reinterpret_cast<float *>(hw.data())[2 * m + 1] = (float)w[m].im;
     }
   }
   if (hipMalloc(&b.chirp, hc.size()) != hipSuccess || hipMalloc(&b.bhat, hw.size()) != hipSuccess)
     return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(Bluestein tables)");
   int st = hip_check(hipMemcpy(b.chirp, hc.data(), hc.size(), hipMemcpyHostToDevice), "hipMemcpy");
   if (!st) st = hip_check(hipMemcpy(b.bhat, hw.data(), hw.size(), hipMemcpyHostToDevice), "hipMemcpy");
-  auto res = p->blue.emplace(n, b);
+  auto res = p->blue.emplace(key, b);
   *out = &res.first->second;
   return st;
 }
@@ -462,13 +504,17 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
     const long long C0 = g.io == IO_C2C ? g.C0r : (g.C0r + 1) / 2;
     if (!mixed_shape(*fv, g.n, C0, radices, s))
       return set_error(D2DHIP_ERR_UNSUPPORTED, "mixed kernel: length not covered");
+    const int M = mixed_length(*fv, g.n);
+    if (M != g.n && (st = get_bluestein(p, g.n, M, radices, &bt))) return st;
   } else if (fv) {
     radices = fv->radices;
   } else {
     bool ok = true;
     radices = factor_radices(g.n, ok);
     if (!ok) {  // a prime factor above 17: Bluestein over a power-of-two length
-      if ((st = get_bluestein(p, g.n, &bt))) return st;
+      int M = 1;
+      while (M < 2 * g.n - 1) M *= 2;
+      if ((st = get_bluestein(p, g.n, M, {}, &bt))) return st;
       radices = factor_radices(bt->M, ok);
     }
   }

@@ -1,12 +1,12 @@
-"""The kernels of any length with factors 2-17 (csrc/mixed_impl.h): every
-radix alone, two to five passes, remainders of the tile (columns, real pairs,
-rows past the last butterfly), both kernel classes, against pocketfft and the
+"""The kernels of any length (csrc/mixed_impl.h): every radix alone, two to
+five passes, Bluestein lengths, remainders of the tile (columns, real pairs,
+rows past the last butterfly), the three kernel classes, against pocketfft and the
 general kernel; the packed y / z stages against stage and pack; grouped
 batches against the plans' own calls.
 
 Tolerances: those of test_gpu_fft.py (1e-13 FP64, 5e-6 FP32, relative L2); a
 transform of n points takes at most log2(n) + 1 rounding steps more than the
-sum, here below 14 of 1.1e-16 (6e-8)."""
+sum, here below 14 (28 for a convolution) of 1.1e-16 (6e-8)."""
 import numpy as np
 import pytest
 
@@ -16,9 +16,11 @@ pytestmark = pytest.mark.gpu
 
 TOL = {64: 1e-13, 32: 5e-6}
 # lengths: each radix, its product with others, 4- and 5-pass schedules,
-# lengths whose tile is one column wide, both classes
+# lengths whose tile is one column wide; then lengths with a prime factor
+# above 17 (two- to four-pass convolutions, the shortest and the longest)
 LENGTHS = [2, 3, 5, 7, 9, 11, 13, 15, 16, 17, 18, 25, 34, 49, 63, 81, 121, 143, 169, 187, 243, 289,
-           375, 405, 450, 625, 686, 729, 1001, 1210, 1875, 2187, 2401, 3125, 4375]
+           375, 405, 450, 625, 686, 729, 1001, 1210, 1875, 2187, 2401, 3125, 4375,
+           19, 23, 29, 41, 62, 107, 191, 247, 382, 509, 638, 1021, 1531, 3067]
 
 
 def dev(torch, a, dt):
@@ -96,7 +98,7 @@ def test_mixed_aligned_and_unaligned_pairs(d2d, torch_gpu):
 
 
 @pytest.mark.parametrize("prec", [64, 32])
-@pytest.mark.parametrize("shape", [(50, 90, 63), (30, 187, 26)])
+@pytest.mark.parametrize("shape", [(50, 90, 63), (30, 187, 26), (18, 57, 101)])
 def test_mixed_packed_stages(d2d, torch_gpu, shape, prec):
     """The default kernels of a rank of a 3 x 2 grid whose lengths have no
     compiled tile: y and z stages fused with pack and unpack equal the stage
