@@ -51,6 +51,23 @@ __device__ __forceinline__ void gstore_r(void *base, long long i, T v) {
   ((D2D_GLOBAL T *)base)[i] = v;
 }
 
+// Two adjacent reals at any multiple of a real (global accesses need no more
+// alignment than that on gfx950).
+template <typename T>
+using gpair = T __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+template <typename T>
+__device__ __forceinline__ cpx<T> gload_pair(const void *base, long long i) {
+  const gpair<T> v = *(const D2D_GLOBAL gpair<T> *)((const D2D_GLOBAL T *)base + i);
+  return cpx<T>{v.x, v.y};
+}
+template <typename T>
+__device__ __forceinline__ void gstore_pair(void *base, long long i, cpx<T> c) {
+  gpair<T> v;
+  v.x = c.x;
+  v.y = c.y;
+  *(D2D_GLOBAL gpair<T> *)((D2D_GLOBAL T *)base + i) = v;
+}
+
 template <typename T>
 __device__ __forceinline__ cpx<T> cadd(cpx<T> a, cpx<T> b) {
   return {a.x + b.x, a.y + b.y};

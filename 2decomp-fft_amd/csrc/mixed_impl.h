@@ -29,12 +29,18 @@
 // vector units are busy 40 % of the time, the twiddle, chirp and spectrum
 // loads keep the address unit busy half of it.  Radices end at 12, where
 // FP64 still fits 128 VGPRs with a pass's twiddles loaded ahead.
+// Real-to-real stages (columns / lines, the general kernel -> here): DCT-II of
+// 300 points 1.2 / 1.3 -> 3.9 / 3.7 TB/s, DCT-I 0.9 / 0.9 -> 2.8 / 2.9, DCT-IV 0.3 /
+// 0.3 -> 3.3 / 3.5; on 513-point grids the compiled DCT-I tiles ran at 2.0 / 2.1
+// where these reach 2.5 / 2.7, the DCT-IV ones at 2.7 / 2.8 against 3.7 / 3.9.
 // What bounds the Stockham classes: up to 600 points the HBM rate of the access pattern; longer
 // columns the workgroups per CU, since a tile of 8 columns takes over half
 // of the LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <atomic>
 
 #include "codelets.h"
 #include "fast_kernels.h"
@@ -44,12 +50,18 @@ namespace d2dhip {
 
 namespace {
 
-// Butterflies of radix R that a lane takes per pass: one, or as many as make
-// 10 values (at most 4).
-constexpr int mx_nb(int r) { return r > 5 ? 1 : (10 / r < 4 ? 10 / r : 4); }
+// Butterflies of radix r that a lane takes per pass: one, or as many as make
+// 10 values, 20 of FP32 columns (at most 4).  (20 FP32 values: columns of 450
+// points 4.7 -> 5.2 TB/s, 675 3.4 -> 5.1; lines of 405 points 4.3 -> 3.5.)
+constexpr int mx_nb(int r, int rb, bool lines) {
+  const int per = (rb == 4 && !lines ? 20 : 10) / r;
+  return per < 1 ? 1 : (per < 4 ? per : 4);
+}
 
 // Radices by kernel class: 0 the codelets that fit 128 VGPRs in FP64 at 1024
-// threads, 1 the large primes too (512 threads), 2 (chirp) those of 0.
+// threads, 1 the large primes too (512 threads), 2 (chirp) those of 0 up to 12,
+// which real-to-real stages take as well.
+constexpr int mx_set(int cls, int io) { return cls == 0 && io == IO_R2R ? 2 : cls; }
 template <int CLS, class F>
 __device__ __forceinline__ void radix_case(int r, F &&f) {
   switch (r) {
@@ -94,7 +106,17 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
                                            long long tile) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   cpx<T> *lds = reinterpret_cast<cpx<T> *>(lds_raw);
-  constexpr bool PAIRED = IO == IO_R2C || IO == IO_C2R;
+  constexpr bool R2R = IO == IO_R2R;
+  constexpr int SET = mx_set(CLS, IO);
+  // real-to-real stages: the transform, and which of its ends are not the
+  // points of the DFT themselves (types 3 and 7 merge the line into a Hermitian
+  // sequence first, 2, 6 and odd-length 4, 8 split the result afterwards);
+  // types 4 and 8 of even length take one real line per tile column
+  const int type = R2R ? d->dtt : 0, Lr = R2R ? d->dtt_len : 0;
+  const bool t48 = type == 4 || type == 8, single = t48 && Lr % 2 == 0;
+  const bool pre = type == 3 || type == 7, post = type == 2 || type == 6 || (t48 && Lr % 2 != 0);
+  const bool alt = type >= 6;  // 6, 7, 8: signs (-1)^j
+  const bool PAIRED = IO == IO_R2C || IO == IO_C2R || (R2R && !single);
   constexpr bool CHIRP = CLS == 2;
   // n: points of a line; m: points of the transform
   const int m = d->n, n = CHIRP ? d->nblue : m, TX = d->TX, lg = d->log2TX, rows = d->rows, np = d->npass;
@@ -114,10 +136,12 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   // lanes without a column or a row take no butterfly (they keep to the barriers)
   if (t >= TX || row >= rows || ca >= (PAIRED ? d->C0r : d->C0)) row = 1 << 24;
   const bool two = !PAIRED || ca + 1 < d->C0r;
+  const bool full = 2 * (c0b + TX) <= d->C0r;  // every pair of the tile is whole
   const long long sji = d->in_sj, sjo = d->out_sj;
-  const long long in_base = (IO == IO_R2C ? ca : c0) * d->in_s0 + c1 * d->in_s1 +
+  const long long f0 = R2R ? d->dtt_first : 0;
+  const long long in_base = (IO == IO_R2C || R2R ? ca : c0) * d->in_s0 + c1 * d->in_s1 + f0 * sji +
                             (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->in_b0 : 0);
-  const long long out_base = (IO == IO_C2R ? ca : c0) * d->out_s0 + c1 * d->out_s1 +
+  const long long out_base = (IO == IO_C2R || R2R ? ca : c0) * d->out_s0 + c1 * d->out_s1 + f0 * sjo +
                              (IO == IO_C2C && !LINES ? (c0 >> d->bsh) * d->out_b0 : 0);
   // LDS: [point][column] for strided columns; [line][point] with one pad
   // point in 17 for contiguous lines, whose first exchange writes with the
@@ -127,25 +151,87 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     return LINES ? j + (j >> 4) + tt * ldt : (j << lg) + tt;
   };
 
+  const bool adj_in = !LINES && d->in_s0 == 1, adj_out = !LINES && d->out_s0 == 1;
+
   // ---- pieces of a pass ------------------------------------------------------
   // values of the first pass (and whole transforms of one pass) from HBM
   auto load = [&](auto rc, auto &v) __attribute__((always_inline)) {
-    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
     const int nb = m / R;
     const long long step = (long long)nb * sji;
-    if constexpr (IO == IO_R2C) {
-      // adjacent columns whose pairs are aligned: one load per pair
-      const bool vec = !LINES && d->in_s0 == 1 && ((sji | d->in_s1) & 1) == 0 &&
-                       ((unsigned long long)in & (sizeof(cpx<T>) - 1)) == 0;
+    if constexpr (R2R) {
+      // point J of the sequence that the DFT takes, types 1, 2, 4, 5, 6, 8: +- x_src
+      // (zero where src is no point of the line), src piecewise linear in J:
+      //   2, 6  x_0 x_2 x_4 ... x_5 x_3 x_1       1  e[j] = e[n-j] = x_j
+      //   5     e[j+1] = -e[n-j-1] = x_j          odd 4, 8  x_j, then zeros
+      // and (x_2J, x_{L-1-2J}) for even 4, 8.  All loads first, then the signs.
+      const int h = (type == 2 || type == 6) ? (n + 1) / 2 : type == 1 ? Lr : type == 5 ? Lr + 1 : n;
+      const int a1 = (type == 2 || type == 6 || single) ? 2 : 1, b1 = type == 5 ? -1 : 0;
+      const int a2 = (type == 2 || type == 6) ? -2 : -1, b2 = (type == 2 || type == 6) ? 2 * n - 1 : type == 1 ? n : n - 1;
+      auto src = [&](int J) __attribute__((always_inline)) {
+        return J < h ? a1 * J + b1 : (CHIRP && J >= n ? -1 : a2 * J + b2);
+      };
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int b = row + q * rows;
+        if (b < nb) {
+          auto off = [&](int s) __attribute__((always_inline)) {
+            const int j = src(b + s * nb);
+            return in_base + (long long)((unsigned)j < (unsigned)Lr ? j : 0) * sji;
+          };
+          if (single) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              v[q * R + s].x = gload_r<T>(in, off(s));
+              const int j = src(b + s * nb);
+              v[q * R + s].y = gload_r<T>(in, in_base + (long long)((unsigned)j < (unsigned)Lr ? 2 * n - 1 - j : 0) * sji);
+            }
+          } else if (adj_in && full) {
+#pragma unroll
+            for (int s = 0; s < R; ++s) v[q * R + s] = gload_pair<T>(in, off(s));
+          } else {
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              v[q * R + s].x = gload_r<T>(in, off(s));
+              v[q * R + s].y = two ? gload_r<T>(in, off(s) + d->in_s0) : T(0);
+            }
+          }
+          if (single) {
+            if (alt) {
+#pragma unroll
+              for (int s = 0; s < R; ++s) v[q * R + s].y = -v[q * R + s].y;
+            }
+          } else if (alt) {
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+              if (src(b + s * nb) & 1) v[q * R + s] = cpx<T>{-v[q * R + s].x, -v[q * R + s].y};
+          } else if (type == 5) {
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+              if (b + s * nb >= h) v[q * R + s] = cpx<T>{-v[q * R + s].x, -v[q * R + s].y};
+          }
+          if (CHIRP || type == 5 || (t48 && !single)) {
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+              if ((unsigned)src(b + s * nb) >= (unsigned)Lr) v[q * R + s] = cpx<T>{T(0), T(0)};
+          }
+          if (t48) {  // exp(-i pi (4J+1) / 4L) of even L, exp(-i pi J / 2L) of odd L
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+              if (b + s * nb < (single ? n : Lr)) v[q * R + s] = cmul(v[q * R + s], gload<T>(d->dtw, b + s * nb));
+          }
+        }
+      }
+    } else if constexpr (IO == IO_R2C) {
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         const int b = row + q * rows;
         if (b < nb) {
           const long long o = in_base + (long long)b * sji;
-          if (vec && two) {
+          if (adj_in && full) {  // adjacent columns: one load per pair
 #pragma unroll
             for (int s = 0; s < R; ++s)
-              if (!CHIRP || b + s * nb < n) v[q * R + s] = gload<T>(in, (o + s * step) >> 1);
+              if (!CHIRP || b + s * nb < n) v[q * R + s] = gload_pair<T>(in, o + s * step);
           } else {
 #pragma unroll
             for (int s = 0; s < R; ++s) {
@@ -188,7 +274,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   };
   // outputs j = b + s * (n / R) of the last pass to HBM
   auto store = [&](auto rc, auto &v) __attribute__((always_inline)) {
-    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
     const int nb = m / R;
     const long long step = (long long)nb * sjo;
 #pragma unroll
@@ -196,12 +282,47 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       const int b = row + q * rows;
       if (b < nb) {
         const long long o = out_base + (long long)b * sjo;
-        if constexpr (IO == IO_C2R) {  // the pre-phase stored conj(Z): z = conj(result)
+        if constexpr (R2R) {  // types 1, 3, 4 and 8 (even length), 5, 7
+          if (single) {  // u_k = V_k exp(-i pi k / L): Y_2k = 2 Re u_k, Y_{L-1-2k} = -2 Im u_k
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              const int J = b + s * nb;
+              if (CHIRP && J >= n) continue;
+              const cpx<T> u = cmul(v[q * R + s], gload<T>(d->dtw, n + J));
+              const int ie = alt ? 2 * n - 1 - 2 * J : 2 * J, io = 2 * n - 1 - ie;
+              gstore_r<T>(out, out_base + (long long)ie * sjo, T(2) * u.x);
+              gstore_r<T>(out, out_base + (long long)io * sjo, T(-2) * u.y);
+            }
+          } else {
+            // 3, 7: z = conj(result) = v_a + i v_b, y_2n = v_n, y_{2n+1} = v_{L-1-n};
+            // 1: the real DFT of an even extension; 5: the imaginary one of an odd
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              const int J = b + s * nb;
+              const cpx<T> z = v[q * R + s];
+              const int kk = pre ? (2 * J < n ? 2 * J : 2 * n - 1 - 2 * J) : type == 1 ? J : J - 1;
+              cpx<T> y = pre ? cconj(z) : type == 1 ? z : cpx<T>{-z.y, z.x};
+              if (pre && alt && (kk & 1)) y = cpx<T>{-y.x, -y.y};
+              if ((unsigned)kk >= (unsigned)Lr || (CHIRP && J >= n)) continue;
+              const long long ok = out_base + (long long)kk * sjo;
+              if (adj_out && full) {
+                gstore_pair<T>(out, ok, y);
+              } else {
+                gstore_r<T>(out, ok, y.x);
+                if (two) gstore_r<T>(out, ok + d->out_s0, y.y);
+              }
+            }
+          }
+        } else if constexpr (IO == IO_C2R) {  // the pre-phase stored conj(Z): z = conj(result)
 #pragma unroll
           for (int s = 0; s < R; ++s) {
             if (CHIRP && b + s * nb >= n) continue;
-            gstore_r<T>(out, o + s * step, v[q * R + s].x);
-            if (two) gstore_r<T>(out, o + s * step + d->out_s0, -v[q * R + s].y);
+            if (adj_out && full) {
+              gstore_pair<T>(out, o + s * step, cconj(v[q * R + s]));
+            } else {
+              gstore_r<T>(out, o + s * step, v[q * R + s].x);
+              if (two) gstore_r<T>(out, o + s * step + d->out_s0, -v[q * R + s].y);
+            }
           }
         } else {
           if (conj) {
@@ -231,13 +352,30 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   };
   // inputs j = b + s * (n / R) of a pass from LDS
   auto lds_read = [&](auto rc, auto &v, int nb, int row_, int rows_, int t_) __attribute__((always_inline)) {
-    constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       const int b = row_ + q * rows_;
       if (b < nb) {
 #pragma unroll
         for (int s = 0; s < R; ++s) v[q * R + s] = lds[A(b + s * nb, t_)];
+      }
+    }
+  };
+
+  // the points outside [dtt_first, dtt_first + dtt_len) of a real-to-real stage
+  auto copy_through = [&]() __attribute__((always_inline)) {
+    if constexpr (R2R) {
+      const int npt = d->dtt_n - Lr, fi = d->dtt_first, per = single ? 1 : 2;
+      for (int w = tid; w < TX * npt; w += nthr) {
+        const int tt = LINES ? w / npt : w & (TX - 1), i = LINES ? w % npt : w >> lg;
+        const int k = i < fi ? i : i + Lr;
+        for (int e = 0; e < per; ++e) {
+          const long long cc = per * (c0b + tt) + e;
+          if (cc < d->C0r)
+            gstore_r<T>(out, cc * d->out_s0 + c1 * d->out_s1 + (long long)k * d->out_sj,
+                        gload_r<T>(in, cc * d->in_s0 + c1 * d->in_s1 + (long long)k * d->in_sj));
+        }
       }
     }
   };
@@ -290,17 +428,78 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     __syncthreads();
   }
 
+  if constexpr (R2R) {
+    if (pre) {
+      // conj(Z_j) = w_j conj(u_j), u_j = (Xa_j + Xb_{L-j}, Xb_j - Xa_{L-j}) (X_L =
+      // 0; DST-III reads X backwards), for j and L - j together
+      constexpr int U = 4;
+      const int nj = n / 2 + 1, total = TX * nj;
+      const float inv_nj = 1.0f / (float)nj;
+      for (int w0 = tid; w0 < total; w0 += U * nthr) {
+        cpx<T> a[U], b[U];
+        int jj[U], tt[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int w = w0 + u * nthr;
+          jj[u] = -1;
+          tt[u] = 0;
+          a[u] = b[u] = cpx<T>{T(0), T(0)};
+          if (w < total) {
+            if constexpr (LINES) {
+              est_divmod(w, nj, inv_nj, tt[u], jj[u]);
+            } else {
+              tt[u] = w & (TX - 1);
+              jj[u] = w >> lg;
+            }
+            const int j = jj[u];
+            const long long cc = 2 * (c0b + tt[u]);
+            const long long base = cc * d->in_s0 + c1 * d->in_s1 + f0 * sji;
+            const long long o1 = base + (long long)(alt ? n - 1 - j : j) * sji;
+            const long long o2 = base + (long long)(alt ? j - 1 : n - j) * sji;
+            if (cc + 1 < d->C0r && adj_in) {
+              a[u] = gload_pair<T>(in, o1);
+              if (j > 0) b[u] = gload_pair<T>(in, o2);
+            } else if (cc < d->C0r) {
+              a[u].x = gload_r<T>(in, o1);
+              if (j > 0) b[u].x = gload_r<T>(in, o2);
+              if (cc + 1 < d->C0r) {
+                a[u].y = gload_r<T>(in, o1 + d->in_s0);
+                if (j > 0) b[u].y = gload_r<T>(in, o2 + d->in_s0);
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int j = jj[u], jm = n - j;
+          if (j >= 0) {
+            const cpx<T> cs = gload<T>(d->dtw, j);
+            const T ux = a[u].x + b[u].y, uy = a[u].y - b[u].x;
+            lds[A(j, tt[u])] = cpx<T>{cs.x * ux - cs.y * uy, -(cs.x * uy + cs.y * ux)};
+            if (j > 0 && j < jm) {
+              const cpx<T> cm = gload<T>(d->dtw, jm);
+              const T vx = b[u].x + a[u].y, vy = b[u].y - a[u].x;
+              lds[A(jm, tt[u])] = cpx<T>{cm.x * vx - cm.y * vy, -(cm.x * vy + cm.y * vx)};
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+
   // ---- passes --------------------------------------------------------------------
-  constexpr bool HBM_IN = IO != IO_C2R, HBM_OUT = IO != IO_R2C;
-  if constexpr (HBM_IN && HBM_OUT && !CHIRP) {
-    if (np == 1) {
-      radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
-        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+  const bool HBM_IN = IO != IO_C2R && !pre, HBM_OUT = IO != IO_R2C && !post;
+  if constexpr (!CHIRP) {
+    if (HBM_IN && HBM_OUT && np == 1) {
+      radix_case<SET>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         cpx<T> v[NB * R];
         load(rc, v);
         if (row < rows) dft<T, R>(v);  // n == R: one butterfly per column
         store(rc, v);
       });
+      copy_through();
       return;
     }
   }
@@ -315,13 +514,13 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     // The twiddles of a pass are loaded before its points.
     const T invm = T(1) / (T)m;
     const int tw_last = d->pass[np - 1].tw_off;
-    radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
-      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    radix_case<SET>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
       const int nb = m / R;
       cpx<T> v[NB * R];
 #pragma unroll
       for (int i = 0; i < NB * R; ++i) v[i] = cpx<T>{T(0), T(0)};
-      if constexpr (HBM_IN) {
+      if (HBM_IN) {
         load(rc, v);
       } else {  // the merged spectra, already in LDS
 #pragma unroll
@@ -360,8 +559,8 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       int zero;
       asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
       const int m_ = m + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
-      radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
-        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      radix_case<SET>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         const int nb = m_ / R;
         if (w == turn) {
 #pragma unroll
@@ -411,8 +610,8 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       });
       __syncthreads();
     }
-    radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
-      constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    radix_case<SET>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+      constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
       const int nb = m / R;
       cpx<T> v[NB * R];
 #pragma unroll
@@ -431,18 +630,18 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
             if (b + s * nb < n) {
               const cpx<T> y = cmul(cconj(v[q * R + s]), gload<T>(d->chirp, b + s * nb));
               v[q * R + s] = cpx<T>{y.x * invm, y.y * invm};
-              if constexpr (!HBM_OUT) lds[A(b + s * nb, t)] = v[q * R + s];
+              if (!HBM_OUT) lds[A(b + s * nb, t)] = v[q * R + s];
             }
         }
       }
-      if constexpr (HBM_OUT) store(rc, v);
+      if (HBM_OUT) store(rc, v);
     });
-    if constexpr (!HBM_OUT) __syncthreads();
+    if (!HBM_OUT) __syncthreads();
   } else {
     int p = 0;
-    if constexpr (HBM_IN) {
-      radix_case<CLS>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
-        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+    if (HBM_IN) {
+      radix_case<SET>(d->pass[0].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         const int nb = n / R;
         cpx<T> v[NB * R];
         load(rc, v);
@@ -467,8 +666,8 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       int zero;
       asm volatile("s_mov_b32 %0, 0" : "=s"(zero));
       const int n_ = n + zero, rows_ = rows + zero, row_ = row + zero, t_ = t + zero;
-      radix_case<CLS>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
-        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      radix_case<SET>(d->pass[p].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         const int nb = n_ / R;
         cpx<T> v[NB * R];
         lds_read(rc, v, nb, row_, rows_, t_);
@@ -493,10 +692,10 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       });
       __syncthreads();
     }
-    if constexpr (HBM_OUT) {
+    if (HBM_OUT) {
       const int tw_off = d->pass[np - 1].tw_off;
-      radix_case<CLS>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
-        constexpr int R = decltype(rc)::value, NB = mx_nb(R);
+      radix_case<SET>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
+        constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         const int nb = n / R;  // = L: every butterfly of the last pass is its own k
         cpx<T> v[NB * R];
         lds_read(rc, v, nb, row, rows, t);
@@ -516,7 +715,48 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
       });
     }
   }
-  if constexpr (!HBM_OUT) {
+  if constexpr (R2R) {
+    if (post) {
+      // Z in LDS.  Types 2, 6: Y_k = 2 Re(w_q V_q) of each line of the pair, V
+      // split from Z as in a real-to-complex transform, q = k (DCT-II) or
+      // L-1-k (DST-II).  Types 4, 8 of odd L (n = 2L): zeta_k = exp(-i pi (2k+1)
+      // / 4L) Z_k, Y_a = Re(zeta_k - zeta_{n-1-k}), Y_b the imaginary parts
+      const int total = TX * Lr;
+      const float inv_L = 1.0f / (float)Lr;
+      for (int w = tid; w < total; w += nthr) {
+        int tt, k;
+        if constexpr (LINES) {
+          est_divmod(w, Lr, inv_L, tt, k);
+        } else {
+          tt = w & (TX - 1);
+          k = w >> lg;
+        }
+        const long long cc = 2 * (c0b + tt);
+        if (cc < d->C0r) {
+          const int q = alt ? Lr - 1 - k : k;
+          cpx<T> y;
+          if (t48) {
+            const cpx<T> cw = gload<T>(d->dtw, Lr + q);
+            const cpx<T> z1 = cmul(cw, lds[A(q, tt)]), z2 = cmul(cconj(cw), lds[A(n - 1 - q, tt)]);
+            y = cadd(z1, z2);
+          } else {
+            const cpx<T> zk = lds[A(q, tt)], zm = lds[A(q == 0 ? 0 : n - q, tt)];
+            const cpx<T> cs = gload<T>(d->dtw, q);
+            y = cpx<T>{cs.x * (zk.x + zm.x) + cs.y * (zk.y - zm.y),
+                       cs.x * (zk.y + zm.y) + cs.y * (zm.x - zk.x)};
+          }
+          const long long o = cc * d->out_s0 + c1 * d->out_s1 + (f0 + k) * sjo;
+          if (cc + 1 < d->C0r && adj_out) {
+            gstore_pair<T>(out, o, y);
+          } else {
+            gstore_r<T>(out, o, y.x);
+            if (cc + 1 < d->C0r) gstore_r<T>(out, o + d->out_s0, y.y);
+          }
+        }
+      }
+    }
+    copy_through();
+  } else if constexpr (IO == IO_R2C) {
     // A[k] = (Z[k] + conj Z[n-k]) / 2 and B[k] = (Z[k] - conj Z[n-k]) / (2i)
     const T half = T(0.5);
     const int total = TX * nh;
@@ -601,15 +841,23 @@ int mixed_launch_multi(const MultiGroup *g, int ng, long long tiles, int nt, siz
 
 constexpr int kMaxLds = 160 * 1024;
 
+// The LDS limit of the kernels, raised once per device (a bit of `done`).
 template <typename T, int IO, bool LINES, int CLS>
 hipError_t mixed_prepare() {
-  hipError_t e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, false>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+  static std::atomic<unsigned long long> done{0};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+  if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
+  e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, false>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
   if constexpr (IO == IO_C2C && !LINES) {
     if (e == hipSuccess)
       e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, true>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
   }
+  if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
   return e;
 }
 
@@ -628,14 +876,16 @@ FastVariant mixed_variant(const char *name) {
   return v;
 }
 
-// c2c, r2c and c2r of one class, strided columns and contiguous lines
+// c2c, r2c, c2r and r2r of one class, strided columns and contiguous lines
 #define D2D_MIXED_ALL(T, CLS, TAG)                                            \
   mixed_variant<T, IO_C2C, false, CLS>(#T " mixed c2c" TAG),                  \
       mixed_variant<T, IO_C2C, true, CLS>(#T " mixed c2c" TAG),               \
       mixed_variant<T, IO_R2C, false, CLS>(#T " mixed r2c" TAG),              \
       mixed_variant<T, IO_R2C, true, CLS>(#T " mixed r2c" TAG),               \
       mixed_variant<T, IO_C2R, false, CLS>(#T " mixed c2r" TAG),              \
-      mixed_variant<T, IO_C2R, true, CLS>(#T " mixed c2r" TAG)
+      mixed_variant<T, IO_C2R, true, CLS>(#T " mixed c2r" TAG),               \
+      mixed_variant<T, IO_R2R, false, CLS>(#T " mixed dct" TAG),              \
+      mixed_variant<T, IO_R2R, true, CLS>(#T " mixed dct" TAG)
 
 }  // namespace
 

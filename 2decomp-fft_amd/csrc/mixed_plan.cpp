@@ -14,9 +14,9 @@ constexpr int kRadices[3][15] = {{16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2},
 
 // Least rows per column of a schedule (every pass within its butterflies per
 // lane), and the work of its passes in lanes, idle ones counted.
-int least_rows(int n, const std::vector<int> &r) {
+int least_rows(int n, const std::vector<int> &r, const FastVariant &v) {
   int rows = 1;
-  for (int x : r) rows = std::max(rows, (n / x + mx_nb(x) - 1) / mx_nb(x));
+  for (int x : r) rows = std::max(rows, (n / x + mx_nb(x, v.rb, v.lines) - 1) / mx_nb(x, v.rb, v.lines));
   return rows;
 }
 double sched_cost(int n, int rows, const std::vector<int> &r) {
@@ -27,11 +27,11 @@ double sched_cost(int n, int rows, const std::vector<int> &r) {
 
 // Schedules of n over non-increasing radices, at most 5 passes; keeps the
 // cheapest.
-void search(int n, int left, int from, int cls, std::vector<int> &cur, std::vector<int> &best, int &rows,
+void search(int n, int left, int from, int set, const FastVariant &v, std::vector<int> &cur, std::vector<int> &best, int &rows,
             double &cost) {
   if (left == 1) {
     // the least rows, or up to half as many again where they divide a pass evenly
-    const int r0 = least_rows(n, cur);
+    const int r0 = least_rows(n, cur, v);
     auto take = [&](int r) {
       if (r < r0 || r > r0 + r0 / 2) return;
       const double c = sched_cost(n, r, cur);
@@ -47,11 +47,11 @@ void search(int n, int left, int from, int cls, std::vector<int> &cur, std::vect
     return;
   }
   if (cur.size() == 5) return;
-  for (int i = from; i < 15 && kRadices[cls][i]; ++i) {
-    const int x = kRadices[cls][i];
+  for (int i = from; i < 15 && kRadices[set][i]; ++i) {
+    const int x = kRadices[set][i];
     if (left % x) continue;
     cur.push_back(x);
-    search(n, left / x, i, cls, cur, best, rows, cost);
+    search(n, left / x, i, set, v, cur, best, rows, cost);
     cur.pop_back();
   }
 }
@@ -99,7 +99,7 @@ bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &ra
   std::vector<int> cur;
   double cost = 1e30;
   int rows = 0;
-  search(n, n, 0, cls, cur, radices, rows, cost);
+  search(n, n, 0, mx_set(cls, v.io), v, cur, radices, rows, cost);
   if (!rows) return false;
   if (v.lines)  // an odd first radix: its stride spreads the first exchange over the banks
     std::stable_partition(radices.begin(), radices.end(), [](int x) { return x % 2 == 1; });

@@ -47,7 +47,6 @@ struct StageGeom {
   // transformed points, points per line; n is the extension's length
   int dtt = 0, dtt_first = 0, dtt_len = 0, dtt_n = 0;
   const void *dtw = nullptr;  // half-length types: (cos, sin)(pi k / (2 dtt_len))
-  const void *dtw4 = nullptr;  // DCT-IV / DST-IV on L/2-point tiles: pre- and post-twiddles
 };
 
 // Chirp tables of a Bluestein length.
@@ -487,6 +486,35 @@ int get_bluestein(d2dhip_plan_s *p, int n, int M, const std::vector<int> &order,
   return st;
 }
 
+int get_dtt4_twiddles(d2dhip_plan_s *p, int L, const void **out);
+int get_dtt4_odd_twiddles(d2dhip_plan_s *p, int L, const void **out);
+
+// Points of the DFT that the kernels of any length run a stage through: the
+// line's, or for a real-to-real stage its length L (types 2, 3, 6, 7), the
+// extension's (2(L-1), 2(L+1) for types 1, 5), or for types 4, 8 half of an even
+// L and twice an odd one.
+int stage_dft(const StageGeom &g) {
+  if (g.io != IO_R2R) return g.n;
+  if (g.dtt == 4 || g.dtt == 8) return g.dtt_len % 2 ? 2 * g.dtt_len : g.dtt_len / 2;
+  return g.n;
+}
+
+// Whether the general kernel's tile of length n fits a workgroup: the lengths
+// that a plan takes when no tile is compiled for them.
+int general_fits(const d2dhip_plan_s *p, const StageGeom &g) {
+  bool ok = true;
+  std::vector<int> r = factor_radices(g.n, ok);
+  int M = g.n;
+  if (!ok) {
+    for (M = 1; M < 2 * g.n - 1;) M *= 2;
+    r = factor_radices(M, ok);
+  }
+  std::vector<PassInfo> passes;
+  for (int x : r) passes.push_back(PassInfo{x, 1, 0, 1.0f});
+  AxisShape s;
+  return choose_shape(M, passes, g.axis == 0, 2 * p->rb, (g.C0r + 1) / 2, s);
+}
+
 // Fills the descriptor and launch shape of stage idx for kernel choice c
 // (-1 = general kernel, else the c-th specialised candidate).
 int configure(d2dhip_plan_s *p, int idx, int c) {
@@ -500,12 +528,19 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   const FastVariant *fv = (c >= 0) ? g.cands[c] : nullptr;
   const BlueTables *bt = nullptr;
   int st;
+  const int line = fv && fv->mixed ? stage_dft(g) : g.n;  // points of the stage's DFT
+  const bool t48 = g.dtt == 4 || g.dtt == 8;
+  // tile columns are single lines, not pairs of real ones
+  const bool single = g.io == IO_C2C || (fv && fv->mixed && t48 && g.dtt_len % 2 == 0);
+  const void *dtw = g.dtw;
   if (fv && fv->mixed) {
-    const long long C0 = g.io == IO_C2C ? g.C0r : (g.C0r + 1) / 2;
-    if (!mixed_shape(*fv, g.n, C0, radices, s))
+    if (!mixed_shape(*fv, line, single ? g.C0r : (g.C0r + 1) / 2, radices, s))
       return set_error(D2DHIP_ERR_UNSUPPORTED, "mixed kernel: length not covered");
-    const int M = mixed_length(*fv, g.n);
-    if (M != g.n && (st = get_bluestein(p, g.n, M, radices, &bt))) return st;
+    const int M = mixed_length(*fv, line);
+    if (M != line && (st = get_bluestein(p, line, M, radices, &bt))) return st;
+    if (t48 && (st = g.dtt_len % 2 ? get_dtt4_odd_twiddles(p, g.dtt_len, &dtw)
+                                   : get_dtt4_twiddles(p, g.dtt_len, &dtw)))
+      return st;
   } else if (fv) {
     radices = fv->radices;
   } else {
@@ -522,17 +557,17 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   st = get_twiddles(p, radices, &tt);
   if (st) return st;
   a.tw = tt->d;
-  a.n = fv && !fv->mixed ? fv->n : (bt ? bt->M : g.n);
+  a.n = fv && !fv->mixed ? fv->n : (bt ? bt->M : line);
   if (bt) {
     a.blue = 1;
-    a.nblue = g.n;
+    a.nblue = line;
     a.chirp = bt->chirp;
     a.bhat = bt->bhat;
   }
   a.npass = (int)tt->passes.size();
   for (int i = 0; i < a.npass; ++i) a.pass[i] = tt->passes[i];
   a.C0r = g.C0r;
-  a.C0 = (g.io == IO_C2C || (fv && fv->io == IO_DTT4)) ? g.C0r : (g.C0r + 1) / 2;
+  a.C0 = single ? g.C0r : (g.C0r + 1) / 2;
   a.C1 = g.C1;
   if (fv) {
     if (!fv->mixed) {
@@ -569,7 +604,7 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   a.dtt_first = g.dtt_first;
   a.dtt_len = g.dtt_len;
   a.dtt_n = g.dtt_n;
-  a.dtw = (fv && fv->io == IO_DTT4) ? g.dtw4 : g.dtw;
+  a.dtw = dtw;
   p->fast[idx] = fv;
   g.choice = c;
   return D2DHIP_SUCCESS;
@@ -610,6 +645,10 @@ int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, 
       for (const FastVariant &v : fast_registry())
         if (v.mixed && v.rb == p->rb && v.io == io && v.lines == (axis == 0 ? 1 : 0) && mixed_runs(v, g.n))
           g.cands.push_back(&v);
+  }
+  if (!g.cands.empty() && g.cands[0]->mixed) {
+    const int st = general_fits(p, g);
+    if (st) return st;
   }
   return configure(p, idx, g.cands.empty() ? -1 : 0);
 }
@@ -674,6 +713,38 @@ int get_dtt4_twiddles(d2dhip_plan_s *p, int L, const void **out) {
   return hip_check(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice), "hipMemcpy");
 }
 
+// exp(-i pi j / (2L)), j < L, then exp(-i pi (2k+1) / (4L)), k < L: the pre- and
+// post-twiddles of DCT-IV / DST-IV of odd L through a DFT of 2L points (kept
+// under key -L, which only odd lengths use for it).
+int get_dtt4_odd_twiddles(d2dhip_plan_s *p, int L, const void **out) {
+  auto it = p->dtw.find(-L);
+  if (it != p->dtw.end()) {
+    *out = it->second;
+    return D2DHIP_SUCCESS;
+  }
+  const int rb = p->rb;
+  std::vector<unsigned char> h((size_t)L * 4 * rb);
+  for (int k = 0; k < 2 * L; ++k) {
+    long double c, s;
+    if (k < L)
+      unit_root(k, 4LL * L, c, s);
+    else
+      unit_root(2LL * (k - L) + 1, 8LL * L, c, s);
+    if (rb == 8) {
+      reinterpret_cast<double *>(h.data())[2 * k] = (double)c;
+      reinterpret_cast<double *>(h.data())[2 * k + 1] = (double)-s;
+    } else {
+      reinterpret_cast<float *>(h.data())[2 * k] = (float)c;
+      reinterpret_cast<float *>(h.data())[2 * k + 1] = (float)-s;
+    }
+  }
+  void *d = nullptr;
+  if (hipMalloc(&d, h.size()) != hipSuccess) return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(DTT twiddles)");
+  p->dtw[-L] = d;
+  *out = d;
+  return hip_check(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice), "hipMemcpy");
+}
+
 // A real-to-real stage along `axis` of the (nx,ny,nz) real array, in place
 // or not (same layout on both sides): `len` points from `first` (0-based) of
 // every line go through a transform of `type`, computed through a DFT of
@@ -685,7 +756,6 @@ int make_dtt_stage(d2dhip_plan_s *p, int idx, int axis, int type, int first, int
   g.axis = axis;
   g.io = IO_R2R;
   g.dtw = nullptr;
-  g.dtw4 = nullptr;
   switch (type) {
     case 1: g.n = 2 * (len - 1); break;
     case 5: g.n = 2 * (len + 1); break;
@@ -713,19 +783,22 @@ int make_dtt_stage(d2dhip_plan_s *p, int idx, int axis, int type, int first, int
   g.dtt_n = axis == 0 ? p->nx : (axis == 1 ? p->ny : p->nz);
   if (!std::getenv("D2DHIP_NO_FAST")) {  // specialised tiles of the stage's DFT length
     const int lines = axis == 0 ? 1 : 0;
-    if ((type == 4 || type == 8) && len % 2 == 0) {  // first choice: L/2-point tiles
-      for (const FastVariant &v : fast_registry())
-        if (v.rb == p->rb && v.mf == 0 && v.io == IO_DTT4 && v.lines == lines && v.n == len / 2)
-          g.cands.push_back(&v);
-      if (!g.cands.empty()) {
-        const int st = get_dtt4_twiddles(p, len, &g.dtw4);
-        if (st) return st;
-      }
-    }
     const int want = (type == 2 || type == 6) ? IO_DTT2 : (type == 3 || type == 7) ? IO_DTT3 : IO_DTTX;
+    if (type != 4 && type != 8)
+      for (const FastVariant &v : fast_registry())
+        if (v.rb == p->rb && v.mf == 0 && v.io == want && v.lines == lines && v.n == g.n)
+          g.cands.push_back(&v);
+    // then the kernels of any length, from DFTs of 16 points (shorter ones are
+    // all launch and load latency: the general kernel is as fast), or of 4 for
+    // types 4 and 8, whose DFT is 4 to 16 times longer on the general kernel
+    const int nd = stage_dft(g), least = type == 4 || type == 8 ? 4 : 16;
     for (const FastVariant &v : fast_registry())
-      if (v.rb == p->rb && v.mf == 0 && v.io == want && v.lines == lines && v.n == g.n)
+      if (nd >= least && v.mixed && v.rb == p->rb && v.io == IO_R2R && v.lines == lines && mixed_runs(v, nd))
         g.cands.push_back(&v);
+  }
+  if (!g.cands.empty() && g.cands[0]->mixed) {
+    const int st = general_fits(p, g);
+    if (st) return st;
   }
   return configure(p, idx, g.cands.empty() ? -1 : 0);
 }
@@ -1900,7 +1973,8 @@ long long d2dhip_plan_device_bytes(d2dhip_plan p) {
   if (!p) return 0;
   long long b = (long long)p->wk_bytes;
   for (auto &kv : p->tw) b += (long long)kv.second.bytes;
-  for (auto &kv : p->dtw) b += (long long)std::abs(kv.first) * 2 * p->rb;
+  for (auto &kv : p->dtw)  // (odd lengths under a negative key: two entries a point)
+    b += (long long)std::abs(kv.first) * (kv.first < 0 && kv.first % 2 ? 4 : 2) * p->rb;
   return b;
 }
 

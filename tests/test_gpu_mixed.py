@@ -157,3 +157,50 @@ def test_mixed_grouped_batch(d2d, torch_gpu, prec):
         b.check()
         for o, q in zip(outs, seq):
             assert torch.equal(o, q)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n", [18, 32, 33, 46, 64, 65, 91, 100, 123, 244, 405, 482, 513])
+def test_mixed_real_to_real(d2d, oracle, torch_gpu, n, axis, prec):
+    """Every DCT / DST type along one axis of n points (transformed lengths n, n-1
+    and n-2; DFTs of half, once, twice that and Bluestein ones), in place,
+    against the oracle's direct sums and the general kernel.  Tolerances:
+    test_gpu_dtt.py's (1e-13, 2e-6)."""
+    torch = torch_gpu
+    tol = 1e-13 if prec == 64 else 2e-6
+    shape = [5, 4, 3]
+    shape[axis] = n
+    shape = tuple(shape)
+    rdt = np.float64 if prec == 64 else np.float32
+    x = np.asfortranarray(np.random.default_rng(n + axis).uniform(-1, 1, shape).astype(rdt))
+    ran = 0
+    for t in range(1, 9):
+        dtt = [2, 2, 2]
+        dtt[axis] = t
+        skip = [True, True, True]
+        skip[axis] = False
+        e = d2d.FFTEngine(1, *shape, prec=prec, opt_DTT=dtt, skip_xyz=skip)
+        for sign, st in ((-1, 7 + axis), (1, 10 + axis)):
+            want = oracle.dtt3d(x.astype(np.float64), tuple(dtt), sign, 1, skip=tuple(skip))
+            for name in [c for c in e.stage_candidates(st) if "mixed" in c]:
+                e.set_stage_kernel(st, name)
+                buf = dev(torch, x, rdt)
+                e.dtt_3d_r2r(buf, buf, sign)
+                assert rel_l2(host(buf, shape), want) < tol, (t, sign, name)
+                e.set_stage_kernel(st, "general")
+                gen = torch.empty_like(buf)
+                e.dtt_3d_r2r(dev(torch, x, rdt), gen, sign)
+                assert rel_l2(host(buf, shape), host(gen, shape)) < tol, (t, sign, name)
+                ran += 1
+    assert ran >= 14, ran
+
+
+def test_refused_lengths_stay_refused(d2d, torch_gpu):
+    """Stages whose general-kernel tile does not fit a workgroup are refused
+    though a kernel of any length could run them (DCT-IV of 721 points runs on
+    the general kernel through 8 * 721 points, padded to 16384)."""
+    for dtt in ((4, 2, 2), (8, 2, 2)):
+        with pytest.raises(d2d.D2dError):
+            d2d.FFTEngine(1, 722, 4, 3, opt_DTT=dtt)
+    d2d.FFTEngine(1, 722, 4, 3, opt_DTT=(2, 3, 4))
