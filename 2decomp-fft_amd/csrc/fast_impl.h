@@ -121,6 +121,7 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
                           IO != IO_YUP;  // two real columns per tile column
   static_assert(!DTT || XM == 0, "real-to-real stages use the plain exchange");
   const bool cvalid = PAIRED ? (ca < d->C0r) : (c0 < d->C0);
+  const bool full = 2 * (c0b + TX) <= d->C0r;  // (real IO) every pair of the tile is whole
   // real-to-real stages: the transformed points start at dtt_first
   const long long f = DTT ? d->dtt_first : 0;
   // (blocked columns: c2c column stages of the blocked spectral layout)
@@ -335,13 +336,25 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
     }
   } else {
     constexpr int R = RL::r[0], NBR = N / R;
+    if (IO == IO_R2C && !LINES && d->in_s0 == 1 && full) {  // adjacent columns: one load per pair
 #pragma unroll
-    for (int q = 0; q < C::nb(0); ++q) {
-      const int b = r0 + q * RPT;
-      if (C::exact(0) || b < NBR) {
+      for (int q = 0; q < C::nb(0); ++q) {
+        const int b = r0 + q * RPT;
+        if (C::exact(0) || b < NBR) {
 #pragma unroll
-        for (int s = 0; s < R; ++s)
-          v[q * R + s] = fload<T, IO>(d, in, in_base, cvalid, true, ca, b + s * NBR, conj, c1);
+          for (int s = 0; s < R; ++s)
+            v[q * R + s] = gload_pair<T>(in, in_base + (long long)(b + s * NBR) * d->in_sj);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < C::nb(0); ++q) {
+        const int b = r0 + q * RPT;
+        if (C::exact(0) || b < NBR) {
+#pragma unroll
+          for (int s = 0; s < R; ++s)
+            v[q * R + s] = fload<T, IO>(d, in, in_base, cvalid, true, ca, b + s * NBR, conj, c1);
+        }
       }
     }
   }
@@ -580,6 +593,20 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
     }
   } else {
     static_assert(P >= 2, "single-pass lengths go through the general kernel");
+    if (IO == IO_C2R && !LINES && d->out_s0 == 1 && full) {  // adjacent columns: one store per pair
+#pragma unroll
+      for (int q = 0; q < C::nb(P - 1); ++q) {
+        const int b = r0 + q * RPT;
+        if (C::exact(P - 1) || b < NBZ) {
+          const int k = b % LZ, g = b / LZ;
+#pragma unroll
+          for (int s = 0; s < RZ; ++s)
+            gstore_pair<T>(out, out_base + (long long)(g * LZ * RZ + k + s * LZ) * d->out_sj,
+                           cconj(v[q * RZ + s]));
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < C::nb(P - 1); ++q) {
       const int b = SHUF ? kq + 16 * (4 * gq + q) : r0 + q * RPT;

@@ -610,6 +610,38 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   return D2DHIP_SUCCESS;
 }
 
+// Candidate that an untuned stage runs: the first registered tile of its
+// length, with two rules measured on 1.2 GB stages of every registered length
+// (TB/s, compiled tile / any-length kernel).
+// Short lengths of pencils that come from HBM run on the any-length kernels,
+// whose tiles are wider: FP64
+// columns of 64 / 128 / 256 points 4.6 / 4.6 / 4.7 against 5.3 / 5.2 / 5.1 (of 320
+// 4.7 against 4.6), FP32 of 192 / 256 points 3.4 / 4.8 against 5.0 / 5.1 (of 384
+// 4.6 against 4.2); c2r lines of 80 / 96 / 128 / 160 points 3.3 / 3.2 / 4.1 / 4.1
+// against 4.8 / 5.3 / 5.3 / 5.4 (of 192 5.5 against 5.4), r2c lines of 80 / 96
+// points 4.4 / 4.7 against 5.2 / 5.3 (of 128 5.4 against 4.9).  Pencils below
+// 128 MB stay in the memory-side cache, where the compiled tiles' shorter
+// latency counts more (128^3: 12.0 against 12.8 us a stage).
+// r2c columns of 896 points and more run there too (FP64 3.7 against 4.0, 1024
+// points 3.7 against 4.1), other real columns on the first tile that leaves
+// room for a second workgroup on the CU (c2r columns of 1152 points 3.5 on 8
+// columns, 4.3 on 4).
+int default_choice(const d2dhip_plan_s *p, const StageGeom &g) {
+  if (g.cands.empty()) return -1;
+  if (g.cands[0]->mixed || g.cands[0]->mf || g.io == IO_R2R) return 0;
+  const bool f64 = p->rb == 8, lines = g.axis == 0, real = g.io != IO_C2C;
+  const int n_short = !lines ? (real ? 256 : f64 ? 300 : 256)
+                             : (g.io == IO_R2C ? (f64 ? 100 : 192) : 160);
+  const bool cached = g.out_elems * (g.io == IO_C2R ? 1 : 2) * p->rb < (128ll << 20);
+  const bool any = (g.n <= n_short && !cached) || (g.io == IO_R2C && !lines && g.n >= 896);
+  for (size_t c = 0; c < g.cands.size(); ++c)
+    if (any && g.cands[c]->mixed) return (int)c;
+  if (real && !lines)
+    for (size_t c = 0; c < g.cands.size(); ++c)
+      if (!g.cands[c]->mixed && g.cands[c]->lds_bytes <= 80 * 1024) return (int)c;
+  return 0;
+}
+
 int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, long long in_elems,
                long long out_elems) {
   StageGeom &g = p->geom[idx];
@@ -650,7 +682,7 @@ int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, 
     const int st = general_fits(p, g);
     if (st) return st;
   }
-  return configure(p, idx, g.cands.empty() ? -1 : 0);
+  return configure(p, idx, default_choice(p, g));
 }
 
 // (cos, sin)(pi k / (2L)), k < L, in long double rounded to the plan's

@@ -2,7 +2,8 @@
 five passes, Bluestein lengths, remainders of the tile (columns, real pairs,
 rows past the last butterfly), the three kernel classes, against pocketfft and the
 general kernel; the packed y / z stages against stage and pack; grouped
-batches against the plans' own calls.
+batches against the plans' own calls; the compiled tiles' column pairs and the
+default between the two.
 
 Tolerances: those of test_gpu_fft.py (1e-13 FP64, 5e-6 FP32, relative L2); a
 transform of n points takes at most log2(n) + 1 rounding steps more than the
@@ -95,6 +96,43 @@ def test_mixed_aligned_and_unaligned_pairs(d2d, torch_gpu):
         e.fft_r2c(x, sp)
         want = np.fft.rfftn(host(x, shape), axes=(0, 1, 2))
         assert rel_l2(host(sp, (nx, ny, 23)), want) < 1e-13, (nx, ny, off)
+
+
+@pytest.mark.parametrize("n", [64, 720, 1024, 2048])
+@pytest.mark.parametrize("nx,off", [(66, 0), (66, 1), (67, 0), (67, 1)])
+@pytest.mark.parametrize("prec", [64, 32])
+def test_compiled_column_pairs(d2d, torch_gpu, n, nx, off, prec):
+    """r2c and c2r along z on every compiled tile: whole tiles take a pair of
+    adjacent real columns in one access, aligned or not (odd row length, odd
+    base address); the last tile, with columns left over, one by one."""
+    torch = torch_gpu
+    rdt, cdt = (torch.float64, torch.complex128) if prec == 64 else (torch.float32, torch.complex64)
+    shape, ss = (nx, 1, n), (nx, 1, n // 2 + 1)
+    buf = torch.rand(nx * n + 1, dtype=rdt, device="cuda")
+    out = torch.full((nx * n + 2,), 7.0, dtype=rdt, device="cuda")
+    x, back = buf[off:off + nx * n], out[off:off + nx * n]
+    sp = torch.empty(nx * (n // 2 + 1), dtype=cdt, device="cuda")
+    e = d2d.FFTEngine(3, *shape, prec=prec)
+    want = np.fft.rfftn(host(x, shape).astype(np.float64), axes=(0, 1, 2))
+    for r, c in zip(e.stage_candidates("r2c"), e.stage_candidates("c2r")):
+        e.set_stage_kernel("r2c", r)
+        e.set_stage_kernel("c2r", c)
+        e.fft_r2c(x, sp)
+        assert rel_l2(host(sp, ss), want) < TOL[prec], r
+        e.fft_c2r(sp, back)
+        assert rel_l2(host(back, shape) / (nx * n), host(x, shape)) < TOL[prec], c
+        assert out[off + nx * n] == 7.0 and (off == 0 or out[0] == 7.0)
+
+
+def test_default_kernel_by_length_and_size(d2d, torch_gpu):
+    """Short lengths start on the any-length kernels only in pencils that do
+    not stay in the memory-side cache."""
+    small = d2d.FFTEngine(1, 128, 128, 128).stage_kernels()
+    large = d2d.FFTEngine(1, 128, 1024, 1024).stage_kernels()
+    assert "mixed" not in small["c2c_x"] and "mixed" in large["c2c_x"]
+    assert "mixed" not in large["c2c_y"]
+    wide = d2d.FFTEngine(1, 1024, 128, 1024).stage_kernels()
+    assert "mixed" not in small["c2c_y"] and "mixed" in wide["c2c_y"]
 
 
 @pytest.mark.parametrize("prec", [64, 32])
