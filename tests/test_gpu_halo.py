@@ -49,6 +49,33 @@ def test_update_halo_matches_oracle(d2d, oracle, torch_gpu, ename, ipencil, shap
         assert np.array_equal(got, want), per
 
 
+@pytest.mark.parametrize("ename", list(ELEMS))
+@pytest.mark.parametrize("ipencil", [1, 2, 3])
+@pytest.mark.parametrize("shape,level", [((1, 2, 3), 1), ((5, 5, 5), 5), ((127, 3, 2), 2),
+                                         ((1027, 3, 4), 3), ((6, 300, 2), 0)])
+def test_update_halo_row_ends(d2d, oracle, torch_gpu, ename, ipencil, shape, level):
+    """Rows of one 16-byte group to several a thread with cells left over,
+    halos as wide as the pencil, no halo; unaligned bases; copies, so equal
+    bit for bit."""
+    torch = torch_gpu
+    dt = ELEMS[ename]
+    rng = np.random.default_rng(shape[0] + ipencil)
+    x = _rand(rng, shape, dt)
+    hs = oracle.halo_shape(shape, level, ipencil)
+    init = _rand(rng, hs, dt)
+    xin = torch.cat([_dev(torch, x)[:1], _dev(torch, x)])[1:]
+    for per in itertools.product([False, True], repeat=3):
+        s = [shape[a] for a in range(3) if a != ipencil - 1 and per[a]]
+        if s and min(s) < level:
+            continue
+        buf = torch.cat([_dev(torch, init)[:1], _dev(torch, init), _dev(torch, init)[:1]])
+        ends = buf[[0, -1]].clone()
+        d2d.update_halo(getattr(d2d, ename), xin, buf[1:-1], shape, level, ipencil, per)
+        got = buf[1:-1].cpu().numpy().reshape(hs, order="F")
+        assert np.array_equal(got, oracle.update_halo(x, level, ipencil, per, init)), per
+        assert torch.equal(buf[[0, -1]], ends)
+
+
 def test_halo_exchange_in_place_and_errors(d2d, oracle, torch_gpu):
     torch = torch_gpu
     shape, level, ipencil = (32, 24, 20), 2, 2
