@@ -30,10 +30,11 @@ double sched_cost(int n, int rows, const std::vector<int> &r) {
 void search(int n, int left, int from, int set, const FastVariant &v, std::vector<int> &cur, std::vector<int> &best, int &rows,
             double &cost) {
   if (left == 1) {
-    // the least rows, or up to half as many again where they divide a pass evenly
+    // the least rows, or up to half as many again where they divide a pass evenly,
+    // within a workgroup's threads
     const int r0 = least_rows(n, cur, v);
     auto take = [&](int r) {
-      if (r < r0 || r > r0 + r0 / 2) return;
+      if (r < r0 || r > r0 + r0 / 2 || r > mx_threads(v.mixed - 1)) return;
       const double c = sched_cost(n, r, cur);
       if (c < cost - 1e-9 || (c < cost + 1e-9 && best == cur && r < rows)) {
         cost = c;
@@ -56,12 +57,10 @@ void search(int n, int left, int from, int set, const FastVariant &v, std::vecto
   }
 }
 
-}  // namespace
-
 // A class takes the lengths that the lighter one does not, up to six points
 // per thread of a block (the fewest a lane may have in a pass) and one
 // column per tile.
-bool mixed_runs(const FastVariant &v, int n) {
+bool takes_length(const FastVariant &v, int n) {
   const int cls = v.mixed - 1;
   int left = n;
   for (int x : {2, 3, 5, 7}) while (left > 0 && left % x == 0) left /= x;
@@ -70,6 +69,16 @@ bool mixed_runs(const FastVariant &v, int n) {
   if (n < 2 || cls != (smooth ? 0 : left == 1 ? 1 : 2)) return false;
   const int m = mixed_length(v, n);
   return m <= 6 * mx_threads(cls) && (size_t)m * 17 / 16 * 2 * v.rb + 64 <= (size_t)kMaxLds;
+}
+
+}  // namespace
+
+// A length of the kernel's class that some schedule fits into a workgroup; the
+// others keep the general kernel.
+bool mixed_runs(const FastVariant &v, int n) {
+  std::vector<int> radices;
+  AxisShape s;
+  return mixed_shape(v, n, 1, radices, s);
 }
 
 // Length of the transform: n itself, or for a chirp the least m >= 2n - 1
@@ -94,7 +103,7 @@ int mixed_length(const FastVariant &v, int n) {
 // threads lie within 5 %).
 bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &radices, AxisShape &s) {
   const int cls = v.mixed - 1, cb = 2 * v.rb;
-  if (!mixed_runs(v, n)) return false;
+  if (!takes_length(v, n)) return false;
   n = mixed_length(v, n);
   std::vector<int> cur;
   double cost = 1e30;
