@@ -116,8 +116,8 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
   const int r0 = LINES ? tid % RPT : tid / TX;
   const long long c0 = c0b + t;
   const long long ca = 2 * c0;  // first real column of a pair (real IO)
-  constexpr bool DTT = IO == IO_DTT2 || IO == IO_DTT3 || IO == IO_DTTX;
-  constexpr bool PAIRED = IO != IO_C2C && IO != IO_YPK && IO != IO_YUN &&
+  constexpr bool DTT = IO == IO_DTT2 || IO == IO_DTT3 || IO == IO_DTTX || IO == IO_DTT4;
+  constexpr bool PAIRED = IO != IO_C2C && IO != IO_DTT4 && IO != IO_YPK && IO != IO_YUN &&
                           IO != IO_YUP;  // two real columns per tile column
   static_assert(!DTT || XM == 0, "real-to-real stages use the plain exchange");
   const bool cvalid = PAIRED ? (ca < d->C0r) : (c0 < d->C0);
@@ -151,7 +151,29 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
   const int gq = rq / HQ, kq = (wq & 3) + 4 * HQ * (wq >> 2) + 4 * (rq % HQ);
 
   // ---- inputs of pass 0 -------------------------------------------------
-  if constexpr (IO == IO_DTTX) {
+  if constexpr (IO == IO_DTT4) {
+    // v_J = (x_{2J} + i x_{2N-1-2J}) exp(-i pi (4J+1) / (8N)) of one line of 2N
+    // points; DST-IV takes (-1)^j x_j
+    const bool alt = d->dtt == 8;
+    constexpr int R = RL::r[0], NBR = N / R;
+#pragma unroll
+    for (int q = 0; q < C::nb(0); ++q) {
+      const int b = r0 + q * RPT;
+      if (C::exact(0) || b < NBR) {
+#pragma unroll
+        for (int s = 0; s < R; ++s) {
+          const int J = b + s * NBR;
+          cpx<T> x = {T(0), T(0)};
+          if (cvalid) {
+            x.x = gload_r<T>(in, in_base + (long long)(2 * J) * d->in_sj);
+            x.y = gload_r<T>(in, in_base + (long long)(2 * N - 1 - 2 * J) * d->in_sj);
+            if (alt) x.y = -x.y;
+          }
+          v[q * R + s] = cmul(x, gload<T>(d->dtw, J));
+        }
+      }
+    }
+  } else if constexpr (IO == IO_DTTX) {
     // the extension e of the line pair, gathered: e[J] = +-x_src or 0
     const int type = d->dtt, Lx = d->dtt_len;
     constexpr int R = RL::r[0], NBR = N / R;
@@ -474,6 +496,27 @@ __device__ __forceinline__ void fast_tile(DescPtr d, const void *in, void *out,
         }
       }
     }
+  } else if constexpr (IO == IO_DTT4) {
+    // u_k = V_k exp(-i pi k / (2N)); DCT-IV: Y_{2k} = 2 Re u_k, Y_{2N-1-2k} =
+    // -2 Im u_k; DST-IV the same outputs read backwards
+    const bool alt = d->dtt == 8;
+#pragma unroll
+    for (int q = 0; q < C::nb(P - 1); ++q) {
+      const int b = r0 + q * RPT;
+      if (C::exact(P - 1) || b < NBZ) {
+        const int k = b % LZ, g = b / LZ;
+#pragma unroll
+        for (int s = 0; s < RZ; ++s) {
+          const int pv = g * LZ * RZ + k + s * LZ;
+          const cpx<T> u = cmul(v[q * RZ + s], gload<T>(d->dtw, N + pv));
+          const int ie = alt ? 2 * N - 1 - 2 * pv : 2 * pv, io = alt ? 2 * pv : 2 * N - 1 - 2 * pv;
+          if (cvalid) {
+            gstore_r<T>(out, out_base + (long long)ie * d->out_sj, T(2) * u.x);
+            gstore_r<T>(out, out_base + (long long)io * d->out_sj, T(-2) * u.y);
+          }
+        }
+      }
+    }
   } else if constexpr (IO == IO_DTTX) {
     // Y_k from E[p] (E_a + i E_b): DCT-I p = k, DST-I p = k + 1; cosines take
     // (Re, Im), sines (-Im, Re)
@@ -731,10 +774,14 @@ static FastVariant make_variant(const char *name) {
       make_variant<T, N, TX, NT, IO_R2C, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " r2c"), \
       make_variant<T, N, TX, NT, IO_C2R, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " c2r")
 
-// real-to-real stages: DCT-II / DST-II and DCT-III / DST-III of N points
-#define D2D_DTT23(T, N, TX, NT, LINES, RL)                                                  \
+// real-to-real stages: DCT-II / DST-II and DCT-III / DST-III of N points,
+// DCT-I and DST-I through an extension of N points, and DCT-IV / DST-IV of 2N
+// points
+#define D2D_DTT(T, N, TX, NT, LINES, RL)                                                    \
   make_variant<T, N, TX, NT, IO_DTT2, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " dct2"), \
-      make_variant<T, N, TX, NT, IO_DTT3, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " dct3")
+      make_variant<T, N, TX, NT, IO_DTT3, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " dct3"), \
+      make_variant<T, N, TX, NT, IO_DTTX, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " dctx"), \
+      make_variant<T, N, TX, NT, IO_DTT4, LINES, RL>(#T " n=" #N " tx=" #TX " nt=" #NT " dct4")
 
 // the y- / z-pencil stage with its output in pack order (" ypk"), with its
 // input in unpack order (" yun"), and with both (" yup"), twins of the c2c

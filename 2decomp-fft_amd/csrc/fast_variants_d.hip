@@ -6,29 +6,28 @@ namespace d2dhip {
 
 std::vector<FastVariant> fast_variants_d() {
   return {
-    // real-to-real stages of (2^k + 1)-point grids (k = 6..10) that run faster
-    // here than on the kernels of any length (mixed_impl.h), measured on 0.8 GB
-    // stages.  DCT-II / III lines in FP64 (513 points 4.7 / 4.2 against 3.7 / 3.7
-    // TB/s; columns 3.6 / 3.4 against 3.7 / 3.8, so none) and FP32 (513 points
-    // 3.7 / 3.7 against 3.2 / 3.4); FP32 DCT-II / III columns (3.2 / 2.9 against
-    // 2.9 / 2.6); FP32 DCT-I / DST-I columns of 1024-point extensions (1.8
-    // against 1.7).
-    D2D_DTT23(double, 1024, 4, 256, true, R16_16_4),
-    D2D_DTT23(double, 512, 4, 256, true, R8_8_8),
-    D2D_DTT23(double, 256, 4, 64, true, R16_16),
-    D2D_DTT23(double, 128, 8, 64, true, R16_8),
-    D2D_DTT23(double, 64, 16, 128, true, R8_8),
-    D2D_DTT23(float, 1024, 8, 512, false, R16_16_4),
-    D2D_DTT23(float, 1024, 4, 256, true, R16_16_4),
-    D2D_DTT23(float, 512, 16, 512, false, R8_8_8),
-    D2D_DTT23(float, 512, 8, 256, true, R8_8_8),
-    D2D_DTT23(float, 256, 16, 256, false, R16_16),
-    D2D_DTT23(float, 256, 4, 64, true, R16_16),
-    D2D_DTT23(float, 128, 16, 128, false, R16_8),
-    D2D_DTT23(float, 128, 8, 64, true, R16_8),
-    D2D_DTT23(float, 64, 16, 128, false, R8_8),
-    D2D_DTT23(float, 64, 16, 128, true, R8_8),
-    make_variant<float, 1024, 8, 512, IO_DTTX, false, R16_16_4>("float n=1024 tx=8 nt=512 dctx"),
+    // real-to-real stages of (2^k + 1)-point grids (k = 6..10), default up to the
+    // pencil sizes that dtt_choice (plan.cpp) gives
+    D2D_DTT(double, 1024, 4, 256, false, R16_16_4),
+    D2D_DTT(double, 1024, 4, 256, true, R16_16_4),
+    D2D_DTT(double, 512, 8, 512, false, R8_8_8),
+    D2D_DTT(double, 512, 4, 256, true, R8_8_8),
+    D2D_DTT(double, 256, 8, 128, false, R16_16),
+    D2D_DTT(double, 256, 4, 64, true, R16_16),
+    D2D_DTT(double, 128, 8, 64, false, R16_8),
+    D2D_DTT(double, 128, 8, 64, true, R16_8),
+    D2D_DTT(double, 64, 8, 64, false, R8_8),
+    D2D_DTT(double, 64, 16, 128, true, R8_8),
+    D2D_DTT(float, 1024, 8, 512, false, R16_16_4),
+    D2D_DTT(float, 1024, 4, 256, true, R16_16_4),
+    D2D_DTT(float, 512, 16, 512, false, R8_8_8),
+    D2D_DTT(float, 512, 8, 256, true, R8_8_8),
+    D2D_DTT(float, 256, 16, 256, false, R16_16),
+    D2D_DTT(float, 256, 4, 64, true, R16_16),
+    D2D_DTT(float, 128, 16, 128, false, R16_8),
+    D2D_DTT(float, 128, 8, 64, true, R16_8),
+    D2D_DTT(float, 64, 16, 128, false, R8_8),
+    D2D_DTT(float, 64, 16, 128, true, R8_8),
     D2D_VARIANTS(float, 32, 16, 64, false, R8_4),
     D2D_VARIANTS(float, 32, 32, 128, true, R8_4),
     D2D_VARIANTS(float, 48, 16, 64, false, R12_4),

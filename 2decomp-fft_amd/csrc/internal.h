@@ -23,9 +23,10 @@ constexpr int kRegCap = 18;
 // IO_DTT2 / IO_DTT3 / IO_DTTX are the I/O forms of the specialised
 // kernels' real-to-real stages: DCT-II / DST-II (a permuted first pass, a
 // twiddled Hermitian split after the last), DCT-III / DST-III (a twiddled
-// Hermitian merge before the first pass, a permuted last pass) and DCT-I /
-// DST-I (the symmetric extension gathered by the first pass, the outputs
-// picked from the last).
+// Hermitian merge before the first pass, a permuted last pass), DCT-I / DST-I
+// (the symmetric extension gathered by the first pass, the outputs picked from
+// the last) and DCT-IV / DST-IV of even length L as an L/2-point DFT of one
+// line (IO_DTT4: tile columns are single real lines, not pairs).
 // IO_YPK / IO_YUN: a c2c stage on the columns of a y- or z-pencil whose
 // output (YPK) is written in, or whose input (YUN) is read from, the
 // alltoallv buffer order of the pencil's exchange (mem_split_yz /
@@ -35,7 +36,7 @@ constexpr int kRegCap = 18;
 // send order.
 enum IoKind : int {
   IO_C2C = 0, IO_R2C = 1, IO_C2R = 2, IO_R2R = 3, IO_DTT2 = 4, IO_DTT3 = 5, IO_DTTX = 6,
-  IO_YPK = 7, IO_YUN = 8, IO_YUP = 9
+  IO_DTT4 = 7, IO_YPK = 8, IO_YUN = 9, IO_YUP = 10
 };
 
 struct PassInfo {
@@ -105,7 +106,7 @@ struct AxisDesc {
   int dtt, dtt_first, dtt_len, dtt_n;
   // (cos, sin)(pi k / (2 dtt_len)), k < dtt_len: the twiddles of the
   // half-length DCT-II / III and DST-II / III stages (n = dtt_len).  DCT-IV /
-  // DST-IV on the kernels of any length: of even dtt_len, an n = dtt_len / 2
+  // DST-IV: of even dtt_len, an n = dtt_len / 2
   // point DFT of single lines, exp(-i pi (4j+1) / (4 dtt_len)), j < n, then
   // exp(-i pi k / dtt_len), k < n; of odd dtt_len, a DFT of 2 dtt_len points of
   // line pairs, exp(-i pi j / (2 dtt_len)), then exp(-i pi (2k+1) / (4 dtt_len))

@@ -529,7 +529,7 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   const int line = fv && fv->mixed ? stage_dft(g) : g.n;  // points of the stage's DFT
   const bool t48 = g.dtt == 4 || g.dtt == 8;
   // tile columns are single lines, not pairs of real ones
-  const bool single = g.io == IO_C2C || (fv && fv->mixed && t48 && g.dtt_len % 2 == 0);
+  const bool single = g.io == IO_C2C || (fv && (fv->io == IO_DTT4 || (fv->mixed && t48 && g.dtt_len % 2 == 0)));
   const void *dtw = g.dtw;
   if (fv && fv->mixed) {
     if (!mixed_shape(*fv, line, single ? g.C0r : (g.C0r + 1) / 2, radices, s))
@@ -541,6 +541,7 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
       return st;
   } else if (fv) {
     radices = fv->radices;
+    if (fv->io == IO_DTT4 && (st = get_dtt4_twiddles(p, g.dtt_len, &dtw))) return st;
   } else {
     bool ok = true;
     radices = factor_radices(g.n, ok);
@@ -608,6 +609,39 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   return D2DHIP_SUCCESS;
 }
 
+// The same for a real-to-real stage with a compiled tile (its first candidate)
+// and an any-length kernel: the tile's shorter latency against the wider rows of
+// the other, by pencil size.  us, tile / any-length, at 24 and 600 MB:
+//   DCT-II / III lines of 512 points FP64 14 / 18, 272 / 335; FP32 16 / 19, 331 /
+//   391: the tile.  FP64 columns 16 / 18, 359 / 352, of 64 points 13 / 15, 385 /
+//   273: the tile up to 128 MB.  FP32 columns of 1024 points 19 / 28, 505 / 641.
+//   DCT-IV columns of 512 points (half of the line's) FP64 14 / 17, 382 / 374,
+//   FP32 18 / 21, 488 / 449: the tile up to 128 MB, FP32 1024 points 20 / 31,
+//   566 / 708 at every size; lines of 64 points FP64 16 / 18 (40 / 40 at 60 MB),
+//   427 / 346: up to 32 MB.
+//   DCT-I of 128-point extensions, 8 and 24 MB: FP64 lines 9 / 10, 20 / 19: the
+//   tile up to 16 MB; where its passes hold 8 values a lane (64 and 512 points)
+//   up to 128 MB (60 MB, 512 points: 35 / 38).  FP32 columns of 256 points 22 /
+//   27, 521 / 474: up to 128 MB, of 1024 points 27 / 37, 673 / 740 always.
+int dtt_choice(const d2dhip_plan_s *p, const StageGeom &g) {
+  const FastVariant &tile = *g.cands[0];
+  int any = 0;
+  for (size_t c = 1; c < g.cands.size() && !any; ++c)
+    if (g.cands[c]->mixed) any = (int)c;
+  const long long mb = (g.out_elems * p->rb) >> 20;
+  const bool f64 = p->rb == 8, lines = g.axis == 0;
+  const bool f32_1024 = !f64 && !lines && tile.n == 1024;
+  bool keep;
+  if (tile.io == IO_DTT2 || tile.io == IO_DTT3)
+    keep = lines || !f64 || mb < 128;
+  else if (tile.io == IO_DTT4)
+    keep = f32_1024 || mb < (lines ? 32 : 128);
+  else
+    keep = f32_1024 || mb < 16 ||
+           (mb < 128 && (f64 ? *std::max_element(tile.radices.begin(), tile.radices.end()) <= 8 : !lines));
+  return keep ? 0 : any;
+}
+
 // Candidate that an untuned stage runs: the first registered tile of its
 // length, with two rules measured on 1.2 GB stages of every registered length
 // (TB/s, compiled tile / any-length kernel).
@@ -626,7 +660,8 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
 // columns, 4.3 on 4).
 int default_choice(const d2dhip_plan_s *p, const StageGeom &g) {
   if (g.cands.empty()) return -1;
-  if (g.cands[0]->mixed || g.cands[0]->mf || g.io == IO_R2R) return 0;
+  if (g.cands[0]->mixed || g.cands[0]->mf) return 0;
+  if (g.io == IO_R2R) return dtt_choice(p, g);
   const bool f64 = p->rb == 8, lines = g.axis == 0, real = g.io != IO_C2C;
   const int n_short = !lines ? (real ? 256 : f64 ? 300 : 256)
                              : (g.io == IO_R2C ? (f64 ? 100 : 192) : 160);
@@ -813,10 +848,11 @@ int make_dtt_stage(d2dhip_plan_s *p, int idx, int axis, int type, int first, int
   g.dtt_n = axis == 0 ? p->nx : (axis == 1 ? p->ny : p->nz);
   if (!std::getenv("D2DHIP_NO_FAST")) {  // specialised tiles of the stage's DFT length
     const int lines = axis == 0 ? 1 : 0;
-    const int want = (type == 2 || type == 6) ? IO_DTT2 : (type == 3 || type == 7) ? IO_DTT3 : IO_DTTX;
-    if (type != 4 && type != 8)
+    const bool t48 = type == 4 || type == 8;
+    const int want = t48 ? IO_DTT4 : (type == 2 || type == 6) ? IO_DTT2 : (type == 3 || type == 7) ? IO_DTT3 : IO_DTTX;
+    if (!t48 || len % 2 == 0)
       for (const FastVariant &v : fast_registry())
-        if (v.rb == p->rb && v.mf == 0 && v.io == want && v.lines == lines && v.n == g.n)
+        if (v.rb == p->rb && v.mf == 0 && v.io == want && v.lines == lines && v.n == (t48 ? len / 2 : g.n))
           g.cands.push_back(&v);
     // then the kernels of any length, from DFTs of 16 points (shorter ones are
     // all launch and load latency: the general kernel is as fast), or of 4 for
@@ -826,11 +862,13 @@ int make_dtt_stage(d2dhip_plan_s *p, int idx, int axis, int type, int first, int
       if (nd >= least && v.mixed && v.rb == p->rb && v.io == IO_R2R && v.lines == lines && mixed_runs(v, nd))
         g.cands.push_back(&v);
   }
+  // (lengths with a compiled tile need no tile of the general kernel: DCT-IV of
+  // 2048 points would take one of 16384)
   if (!g.cands.empty() && g.cands[0]->mixed) {
     const int st = general_fits(p, g);
     if (st) return st;
   }
-  return configure(p, idx, g.cands.empty() ? -1 : 0);
+  return configure(p, idx, default_choice(p, g));
 }
 
 int upload_chunk_descs(d2dhip_plan_s *p);

@@ -75,3 +75,43 @@ def test_long_real_to_real(d2d, oracle, torch_gpu, types, n, points, axis, prec)
             e.dtt_3d_r2r(xin, out, sign)
             want = oracle.dtt3d(x.astype(np.float64), tuple(dtt), sign, 1, skip=tuple(skip))
             assert rel_l2(host(out, shape), want) < RTOL[prec], (t, sign)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("prec", [64, 32])
+def test_dct4_of_2048_points(d2d, oracle, torch_gpu, axis, prec):
+    """DCT-IV and DST-IV of 2048 points run (the general kernel's tile of eight
+    times the length does not fit a workgroup), on every specialised kernel."""
+    rdt = np.float64 if prec == 64 else np.float32
+    shape = [3, 3, 2]
+    shape[axis] = 2049
+    shape = tuple(shape)
+    x = np.asfortranarray(np.random.default_rng(axis).uniform(-1, 1, shape).astype(rdt))
+    xin = dev(torch_gpu, x, rdt)
+    for t in (4, 8):
+        dtt, skip = [2, 2, 2], [True, True, True]
+        dtt[axis], skip[axis] = t, False
+        e = d2d.FFTEngine(1, *shape, prec=prec, opt_DTT=dtt, skip_xyz=skip)
+        for sign, st in ((-1, 7 + axis), (1, 10 + axis)):
+            want = oracle.dtt3d(x.astype(np.float64), tuple(dtt), sign, 1, skip=tuple(skip))
+            names = [n for n in e.stage_candidates(st) if n != "general"]
+            assert len(names) == 2
+            for name in [None] + names:
+                if name:
+                    e.set_stage_kernel(st, name)
+                out = torch_gpu.empty_like(xin)
+                e.dtt_3d_r2r(xin, out, sign)
+                assert rel_l2(host(out, shape), want) < RTOL[prec], (t, sign, name)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+def test_small_pencils_run_the_compiled_real_to_real_tiles(d2d, torch_gpu, prec):
+    """Pencils of less than 16 MB start on the compiled tile of their length,
+    in every transform kind; large ones on the any-length kernels where those
+    are faster."""
+    for n, types in ((65, (2, 3, 6, 7)), (65, (1,)), (257, (4, 8)), (129, (5,))):
+        for t in types:
+            small = d2d.FFTEngine(1, n, n, 20, prec=prec, opt_DTT=(t, t, 2)).dtt_stage_kernels()
+            assert all("mixed" not in small[s] for s in (7, 8, 10, 11)), (n, t, small)
+    large = d2d.FFTEngine(1, 257, 257, 3000, prec=prec, opt_DTT=(4, 4, 2)).dtt_stage_kernels()
+    assert "mixed" in large[7] and "mixed" in large[8]
