@@ -108,6 +108,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   cpx<T> *lds = reinterpret_cast<cpx<T> *>(lds_raw);
   constexpr bool R2R = IO == IO_R2R;
   constexpr int SET = mx_set(CLS, IO);
+  constexpr int LO = R2R && sizeof(T) == 8 ? 2 : 1;  // form of the butterflies (codelets.h)
   // real-to-real stages: the transform, and which of its ends are not the
   // points of the DFT themselves (types 3 and 7 merge the line into a Hermitian
   // sequence first, 2, 6 and odd-length 4, 8 split the result afterwards);
@@ -496,7 +497,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
         constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
         cpx<T> v[NB * R];
         load(rc, v);
-        if (row < rows) dft<T, R>(v);  // n == R: one butterfly per column
+        if (row < rows) dft<T, R, LO>(v);  // n == R: one butterfly per column
         store(rc, v);
       });
       copy_through();
@@ -538,7 +539,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 #pragma unroll
           for (int s = 0; s < R; ++s)
             if (b + s * nb < n) v[q * R + s] = cmul(v[q * R + s], gload<T>(d->chirp, b + s * nb));
-          dft<T, R>(&v[q * R]);
+          dft<T, R, LO>(&v[q * R]);
           lds[A(b, t)] = v[q * R];
 #pragma unroll
           for (int s = 1; s < R; ++s)
@@ -572,10 +573,10 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
               for (int s = 0; s < R; ++s) f[s] = gload<T>(d->bhat, b * R + s);
 #pragma unroll
               for (int s = 0; s < R; ++s) v[s] = lds[A(b * R + s, t_)];
-              dft<T, R>(v);
+              dft<T, R, LO>(v);
 #pragma unroll
               for (int s = 0; s < R; ++s) v[s] = cconj(cmul(v[s], f[s]));
-              dft<T, R>(v);
+              dft<T, R, LO>(v);
 #pragma unroll
               for (int s = 0; s < R; ++s) lds[A(b * R + s, t_)] = v[s];
             }
@@ -597,7 +598,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 #pragma unroll
                 for (int s = 1; s < R; ++s) v[s] = cmul(v[s], f[s]);
               }
-              dft<T, R>(v);
+              dft<T, R, LO>(v);
               if (w < turn) {
 #pragma unroll
                 for (int s = 1; s < R; ++s) v[s] = cmul(v[s], f[s]);
@@ -624,7 +625,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
           v[q * R] = lds[A(b, t)];
 #pragma unroll
           for (int s = 1; s < R; ++s) v[q * R + s] = cmul(lds[A(b + s * nb, t)], f[s]);
-          dft<T, R>(&v[q * R]);
+          dft<T, R, LO>(&v[q * R]);
 #pragma unroll
           for (int s = 0; s < R; ++s)
             if (b + s * nb < n) {
@@ -649,7 +650,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
         for (int q = 0; q < NB; ++q) {
           const int b = row + q * rows;
           if (b < nb) {
-            dft<T, R>(&v[q * R]);
+            dft<T, R, LO>(&v[q * R]);
 #pragma unroll
             for (int s = 0; s < R; ++s) lds[A(b * R + s, t)] = v[q * R + s];
           }
@@ -683,7 +684,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
               for (int s = 1; s < R; ++s)
                 v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + k * (R - 1) + (s - 1)));
             }
-            dft<T, R>(&v[q * R]);
+            dft<T, R, LO>(&v[q * R]);
             const int jb = g * L * R + k;
 #pragma unroll
             for (int s = 0; s < R; ++s) lds[A(jb + s * L, t_)] = v[q * R + s];
@@ -708,7 +709,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
               for (int s = 1; s < R; ++s)
                 v[q * R + s] = cmul(v[q * R + s], gload<T>(tw, tw_off + b * (R - 1) + (s - 1)));
             }
-            dft<T, R>(&v[q * R]);
+            dft<T, R, LO>(&v[q * R]);
           }
         }
         store(rc, v);

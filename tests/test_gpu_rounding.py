@@ -1,0 +1,87 @@
+"""Rounding errors of the kernels of any length (csrc/mixed_impl.h): against
+the transform in extended precision, the root mean square error is no larger
+than the general kernel's, which ran these lengths before.
+
+The bound of the ratio is 1.03.  Both kernels' arithmetic, followed pass by pass
+on a host in the same precision, gives ratios of 0.90 to 1.02 over these
+lengths; 2e5 points or more leave a sampling error of 0.3 %."""
+import numpy as np
+import pytest
+import scipy.fft as sf
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 1.03
+
+
+def _rms(got, want):
+    d = got.astype(want.dtype) - want
+    return float(np.sqrt((np.abs(d) ** 2).sum() / (np.abs(want) ** 2).sum()))
+
+
+def _kernel_errors(d2d, torch, n, axis, prec):
+    """RMS errors of the c2c stage of n points: (general, any-length)."""
+    m1, m2 = 32, max(4, 200000 // (32 * n))
+    shape = (n, m1, m2) if axis == 0 else (m1, n, m2)
+    rng = np.random.default_rng(n + axis)
+    x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    x = x.astype(np.complex128 if prec == 64 else np.complex64)
+    want = sf.fft(x.astype(np.clongdouble if prec == 64 else np.complex128), axis=axis)
+    xin = torch.from_numpy(x.ravel(order="F").copy()).cuda()
+    out = torch.empty_like(xin)
+    e = d2d.FFTEngine(1, *shape, prec=prec)
+    stage = ("c2c_x", "c2c_y")[axis]
+    names = ["general"] + [c for c in e.stage_candidates(stage) if "mixed" in c]
+    assert len(names) == 2
+    err = []
+    for name in names:
+        e.set_stage_kernel(stage, name)
+        e.exec_1m(stage, xin, out, -1)
+        err.append(_rms(out.cpu().numpy().reshape(shape, order="F"), want))
+    return err
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n", [20, 28, 36, 72, 144, 150, 216, 288, 375, 405, 450, 486, 500, 576, 720, 864, 972,
+                               1000, 1024, 26, 34, 77, 242, 286, 308, 935])
+def test_smooth_lengths(d2d, torch_gpu, n, axis, prec):
+    general, mixed = _kernel_errors(d2d, torch_gpu, n, axis, prec)
+    assert mixed < BOUND * general, (general, mixed)
+
+
+def _dtt_errors(d2d, torch, t, points, axis, prec):
+    """RMS errors of the forward transform t of `points` points: (general,
+    any-length); the points that it leaves out are not counted."""
+    n = points + (0 if t == 1 else 2 if t == 5 else 1)
+    first = 1 if t in (5, 7) else 0
+    m1, m2 = 32, max(4, 200000 // (32 * n))
+    shape = (n, m1, m2) if axis == 0 else (m1, n, m2)
+    cut = [slice(None)] * 3
+    cut[axis] = slice(first, first + points)
+    cut = tuple(cut)
+    x = np.random.default_rng(n + axis + t).standard_normal(shape).astype(np.float64 if prec == 64 else np.float32)
+    wide = x[cut].astype(np.longdouble if prec == 64 else np.float64)
+    want = sf.dct(wide, type=t, axis=axis) if t <= 4 else sf.dst(wide, type=t - 4, axis=axis)
+    xin = torch.from_numpy(x.ravel(order="F").copy()).cuda()
+    out = torch.empty_like(xin)
+    dtt, skip = [2, 2, 2], [True, True, True]
+    dtt[axis], skip[axis] = t, False
+    e = d2d.FFTEngine(1, *shape, prec=prec, opt_DTT=dtt, skip_xyz=skip)
+    names = ["general"] + [c for c in e.stage_candidates(7 + axis) if "mixed" in c]
+    assert len(names) == 2
+    err = []
+    for name in names:
+        e.set_stage_kernel(7 + axis, name)
+        e.dtt_3d_r2r(xin, out, -1)
+        err.append(_rms(out.cpu().numpy().reshape(shape, order="F")[cut], want))
+    return err
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("t,points", [(2, 36), (3, 36), (6, 48), (7, 48), (2, 180), (3, 216), (6, 216), (2, 252),
+                                      (3, 400), (2, 450), (1, 109), (5, 107), (1, 151), (5, 224)])
+def test_real_to_real_smooth_lengths(d2d, torch_gpu, t, points, axis, prec):
+    general, mixed = _dtt_errors(d2d, torch_gpu, t, points, axis, prec)
+    assert mixed < BOUND * general, (general, mixed)
