@@ -49,10 +49,12 @@ int launch_batch_fast(int rb, const BatchQueue &q, int blocks, size_t lds, hipSt
 // The kernels of any length (mixed_impl.h); whether one of them runs length
 // n, the length of its transform (longer than n for Bluestein's algorithm,
 // mixed = 3), and the tile and radix schedule that it takes (C0 tile-level
-// columns).
+// columns).  mixed_short: whether its convolution of length n is shorter than the
+// general kernel's, and less accurate.
 std::vector<FastVariant> mixed_variants();
 bool mixed_runs(const FastVariant &v, int n);
 int mixed_length(const FastVariant &v, int n);
+bool mixed_short(const FastVariant &v, int n);
 bool mixed_shape(const FastVariant &v, int n, long long C0, std::vector<int> &radices, AxisShape &s);
 // The split-BF16 matrix-core variants (mfma_kernels.hip).
 std::vector<FastVariant> mf_variants();

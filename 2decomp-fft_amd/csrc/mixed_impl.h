@@ -22,10 +22,9 @@
 //   n = 405  1.9 / 3.0 / 2.4 -> 4.4 / 4.7 / 4.6
 //   n = 1000 1.3 / 2.0 / 1.6 -> 3.9 / 4.9 / 4.9
 // Class 2 ("chirp") runs lengths with a prime factor above 17 by Bluestein's
-// algorithm over a smooth length m >= 2n - 1, in place (the general kernel
-// pads to a power of two and sweeps the LDS tile twelve times at n = 382):
-// columns of 107 / 191 / 382 / 1021 points 1.0 / 0.8 / 0.8 / 0.9 -> 1.9 / 2.1 /
-// 1.9 / 1.7 TB/s.  It is bound by latency and the texture path: at n = 382 the
+// algorithm over a length m >= 2n - 1 (mixed_length), in place (the general kernel
+// sweeps the LDS tile twelve times at n = 382): columns of 101 / 191 / 382 / 1021
+// points 1.0 / 0.8 / 0.8 / 0.9 -> 2.4 / 2.1 / 1.9 / 1.8 TB/s.  It is bound by latency and the texture path: at n = 382 the
 // vector units are busy 40 % of the time, the twiddle, chirp and spectrum
 // loads keep the address unit busy half of it.  Radices end at 12, where
 // FP64 still fits 128 VGPRs with a pass's twiddles loaded ahead.
@@ -59,28 +58,30 @@ constexpr int mx_nb(int r, int rb, bool lines) {
 }
 
 // Radices by kernel class: 0 the codelets that fit 128 VGPRs in FP64 at 1024
-// threads, 1 the large primes too (512 threads), 2 (chirp) those of 0 up to 12,
-// which real-to-real stages take as well.
-constexpr int mx_set(int cls, int io) { return cls == 0 && io == IO_R2R ? 2 : cls; }
-template <int CLS, class F>
+// threads (real-to-real stages only those up to 12: set 2), 1 the large primes too
+// (512 threads), 2 (chirp) those of the convolution lengths: set 3.
+constexpr int mx_set(int cls, int io) { return cls == 2 ? 3 : cls == 0 && io == IO_R2R ? 2 : cls; }
+template <int SET, class F>
 __device__ __forceinline__ void radix_case(int r, F &&f) {
   switch (r) {
     case 2: f(std::integral_constant<int, 2>{}); break;
-    case 3: f(std::integral_constant<int, 3>{}); break;
     case 4: f(std::integral_constant<int, 4>{}); break;
-    case 5: f(std::integral_constant<int, 5>{}); break;
-    case 6: f(std::integral_constant<int, 6>{}); break;
-    case 7: f(std::integral_constant<int, 7>{}); break;
     case 8: f(std::integral_constant<int, 8>{}); break;
-    case 9: f(std::integral_constant<int, 9>{}); break;
     case 10: f(std::integral_constant<int, 10>{}); break;
     case 12: f(std::integral_constant<int, 12>{}); break;
     default:
-      if constexpr (CLS != 2) {
+      if constexpr (SET != 3) {
+        if (r == 3) f(std::integral_constant<int, 3>{});
+        else if (r == 5) f(std::integral_constant<int, 5>{});
+        else if (r == 6) f(std::integral_constant<int, 6>{});
+        else if (r == 7) f(std::integral_constant<int, 7>{});
+        else if (r == 9) f(std::integral_constant<int, 9>{});
+      }
+      if constexpr (SET < 2) {
         if (r == 15) f(std::integral_constant<int, 15>{});
         else if (r == 16) f(std::integral_constant<int, 16>{});
       }
-      if constexpr (CLS == 1) {
+      if constexpr (SET == 1) {
         if (r == 11) f(std::integral_constant<int, 11>{});
         else if (r == 13) f(std::integral_constant<int, 13>{});
         else if (r == 17) f(std::integral_constant<int, 17>{});
@@ -511,9 +512,9 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     // (as conj(DFT(conj(.)))) from the first to the last by decimation in time,
     // all in place: a lane writes a butterfly back to the points it read.  So
     // an exchange takes one barrier, both transforms share one twiddle table,
-    // and the spectrum stays in the first one's order (bhat is stored in it).
+    // and the spectrum stays in the first one's order (bhat is stored in it, over
+    // m).
     // The twiddles of a pass are loaded before its points.
-    const T invm = T(1) / (T)m;
     const int tw_last = d->pass[np - 1].tw_off;
     radix_case<SET>(d->pass[np - 1].r, [&](auto rc) __attribute__((always_inline)) {
       constexpr int R = decltype(rc)::value, NB = mx_nb(R, sizeof(T), LINES);
@@ -629,8 +630,7 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 #pragma unroll
           for (int s = 0; s < R; ++s)
             if (b + s * nb < n) {
-              const cpx<T> y = cmul(cconj(v[q * R + s]), gload<T>(d->chirp, b + s * nb));
-              v[q * R + s] = cpx<T>{y.x * invm, y.y * invm};
+              v[q * R + s] = cmul(cconj(v[q * R + s]), gload<T>(d->chirp, b + s * nb));
               if (!HBM_OUT) lds[A(b + s * nb, t)] = v[q * R + s];
             }
         }

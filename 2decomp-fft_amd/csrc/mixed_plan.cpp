@@ -8,9 +8,10 @@ namespace d2dhip {
 
 namespace {
 
-constexpr int kRadices[3][15] = {{16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2},
+constexpr int kRadices[4][15] = {{16, 15, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2},
                                  {17, 16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2},
-                                 {12, 10, 9, 8, 7, 6, 5, 4, 3, 2}};
+                                 {12, 10, 9, 8, 7, 6, 5, 4, 3, 2},
+                                 {12, 10, 8, 4, 2}};
 
 // Least rows per column of a schedule (every pass within its butterflies per
 // lane), and the work of its passes in lanes, idle ones counted.
@@ -57,6 +58,15 @@ void search(int n, int left, int from, int set, const FastVariant &v, std::vecto
   }
 }
 
+// Passes of the cheapest schedule of m.
+int passes(int m, const FastVariant &v) {
+  std::vector<int> cur, best;
+  int rows = 0;
+  double cost = 1e30;
+  search(m, m, 0, mx_set(v.mixed - 1, v.io), v, cur, best, rows, cost);
+  return rows ? (int)best.size() : 99;
+}
+
 // A class takes the lengths that the lighter one does not, up to six points
 // per thread of a block (the fewest a lane may have in a pass) and one
 // column per tile.
@@ -81,18 +91,37 @@ bool mixed_runs(const FastVariant &v, int n) {
   return mixed_shape(v, n, 1, radices, s);
 }
 
-// Length of the transform: n itself, or for a chirp the least m >= 2n - 1
-// among 2^k times 1, 3, 5, 9 and 15 (m = 768 runs n = 382 at 1.8 TB/s, 800
-// to 960 at 1.6 to 1.7, 1024 at 1.5).
+// Length of the transform: n itself, or for a chirp the least power of two m >=
+// 2n - 1, or 15/16 of it where that saves a pass (960 = 12 10 8 for 1024 = 8 8 8 2:
+// 382-point columns 1.6 -> 1.9 TB/s in FP64, 1.0 -> 1.2 in FP32).  The rounding errors
+// of a convolution grow as the square root of (2n - 1) / m: 3/4 of the power of
+// two (768 for 382 points, 2.0 TB/s) is up to 12 % further from the exact
+// transform than the general kernel, which takes the power of two.  (120 for
+// 128 would save a pass too, and be 2 to 7 % further off in FP64.)  Lengths whose
+// power of two does not fit a workgroup take the least 2^k times 3, 5 or 9; they
+// run on the general kernel unless chosen (mixed_short).
 int mixed_length(const FastVariant &v, int n) {
   if (v.mixed != 3) return n;
-  int best = 0;
-  for (int f : {1, 3, 5, 9, 15}) {
-    int m = f;
+  int m = 16;
+  while (m < 2 * n - 1) m *= 2;
+  if (m <= 6 * mx_threads(2)) {
+    const int q = m / 16 * 15;
+    return m >= 512 && q >= 2 * n - 1 && passes(q, v) < passes(m, v) ? q : m;
+  }
+  int best = m;
+  for (int f : {3, 5, 9}) {
+    m = f;
     while (m < 2 * n - 1) m *= 2;
-    if (!best || m < best) best = m;
+    best = std::min(best, m);
   }
   return best;
+}
+
+bool mixed_short(const FastVariant &v, int n) {
+  if (v.mixed != 3) return false;
+  int m = 16;
+  while (m < 2 * n - 1) m *= 2;
+  return m > 6 * mx_threads(2);
 }
 
 // Columns: the widest rows (256 bytes at most) that leave room for two

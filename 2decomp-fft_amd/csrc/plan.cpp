@@ -407,8 +407,8 @@ void host_dft(const LdCpx *w, long long st, int n, LdCpx *out, const LdCpx *root
 // wrapped as w[m] = w[M-m] = w_m, evaluated in long double with j^2 reduced
 // mod 2n exactly.  `order`: the radices of a schedule whose transform leaves
 // the spectrum in its in-place order, in which bhat is then stored (position
-// d0 + r0 (d1 + r1 (d2 + ...)) holds frequency d0 M/r0 + d1 M/(r0 r1) + ...);
-// empty: natural order.
+// d0 + r0 (d1 + r1 (d2 + ...)) holds frequency d0 M/r0 + d1 M/(r0 r1) + ...),
+// divided by M; empty: natural order, as it is.
 int get_bluestein(d2dhip_plan_s *p, int n, int M, const std::vector<int> &order, const BlueTables **out) {
   std::vector<int> key = {n, M};
   key.insert(key.end(), order.begin(), order.end());
@@ -452,7 +452,7 @@ int get_bluestein(d2dhip_plan_s *p, int n, int M, const std::vector<int> &order,
         f += q % r * step;
         q /= r;
       }
-      w[pos] = nat[f];
+      w[pos] = {nat[f].re / M, nat[f].im / M};
     }
   }
   const int rb = p->rb;
@@ -609,6 +609,12 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   return D2DHIP_SUCCESS;
 }
 
+// Candidates that run only where a caller chooses them: convolutions shorter
+// than the general kernel's, which are less accurate.
+bool only_chosen(const StageGeom &g, int c) {
+  return c >= 0 && g.cands[c]->mixed && mixed_short(*g.cands[c], stage_dft(g));
+}
+
 // The same for a real-to-real stage with a compiled tile (its first candidate)
 // and an any-length kernel: the tile's shorter latency against the wider rows of
 // the other, by pencil size.  us, tile / any-length, at 24 and 600 MB:
@@ -659,7 +665,7 @@ int dtt_choice(const d2dhip_plan_s *p, const StageGeom &g) {
 // room for a second workgroup on the CU (c2r columns of 1152 points 3.5 on 8
 // columns, 4.3 on 4).
 int default_choice(const d2dhip_plan_s *p, const StageGeom &g) {
-  if (g.cands.empty()) return -1;
+  if (g.cands.empty() || only_chosen(g, 0)) return -1;
   if (g.cands[0]->mixed || g.cands[0]->mf) return 0;
   if (g.io == IO_R2R) return dtt_choice(p, g);
   const bool f64 = p->rb == 8, lines = g.axis == 0, real = g.io != IO_C2C;
@@ -1128,7 +1134,7 @@ int tune_stages(d2dhip_plan_s *p) {
       int c = -1;
       for (size_t k = 0; k < g.cands.size(); ++k)
         if (it->second == g.cands[k]->name) c = (int)k;
-      if (c >= 0 || it->second == "general") {
+      if ((c >= 0 && !only_chosen(g, c)) || it->second == "general") {
         st = configure(p, i, c);
         continue;
       }
@@ -1165,6 +1171,7 @@ int tune_stages(d2dhip_plan_s *p) {
     const int nc = (int)g.cands.size();
     std::vector<float> t(nc + 1, 1e30f);  // t[c + 1]: candidate c, -1 = general
     for (int c = -1; c < nc && !st; ++c) {
+      if (only_chosen(g, c)) continue;
       if (configure(p, i, c)) continue;  // e.g. the general kernel cannot run this length
       st = measure(c, &t[c + 1]);
     }

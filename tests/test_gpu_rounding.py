@@ -50,6 +50,26 @@ def test_smooth_lengths(d2d, torch_gpu, n, axis, prec):
     assert mixed < BOUND * general, (general, mixed)
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n", [19, 23, 31, 38, 57, 62, 87, 101, 123, 149, 191, 233, 254, 307, 382, 458, 509, 573, 638,
+                               764, 1021, 1531, 1902])
+def test_bluestein_lengths(d2d, torch_gpu, n, axis, prec):
+    """Convolutions of the same length as the general kernel's, or 15/16 of it."""
+    general, mixed = _kernel_errors(d2d, torch_gpu, n, axis, prec)
+    assert mixed < BOUND * general, (general, mixed)
+
+
+def test_shorter_convolutions_are_not_the_default(d2d, torch_gpu, tmp_path, monkeypatch):
+    """Lengths whose power of two does not fit a workgroup: the kernel of any
+    length is there to be chosen, untuned and tuned plans run the general one."""
+    monkeypatch.setenv("D2DHIP_TUNE_CACHE", str(tmp_path / "tuning.tsv"))
+    for tune in (False, True):
+        e = d2d.FFTEngine(1, 2062, 4, 4, tune=tune)
+        assert e.stage_kernels()["c2c_x"] == "general"
+        assert any("mixed" in c for c in e.stage_candidates("c2c_x"))
+
+
 def _dtt_errors(d2d, torch, t, points, axis, prec):
     """RMS errors of the forward transform t of `points` points: (general,
     any-length); the points that it leaves out are not counted."""
@@ -83,5 +103,13 @@ def _dtt_errors(d2d, torch, t, points, axis, prec):
 @pytest.mark.parametrize("t,points", [(2, 36), (3, 36), (6, 48), (7, 48), (2, 180), (3, 216), (6, 216), (2, 252),
                                       (3, 400), (2, 450), (1, 109), (5, 107), (1, 151), (5, 224)])
 def test_real_to_real_smooth_lengths(d2d, torch_gpu, t, points, axis, prec):
+    general, mixed = _dtt_errors(d2d, torch_gpu, t, points, axis, prec)
+    assert mixed < BOUND * general, (general, mixed)
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("t,points", [(2, 23), (3, 95), (6, 149), (7, 299), (2, 383), (1, 150), (5, 298), (1, 300)])
+def test_real_to_real_bluestein_lengths(d2d, torch_gpu, t, points, axis, prec):
     general, mixed = _dtt_errors(d2d, torch_gpu, t, points, axis, prec)
     assert mixed < BOUND * general, (general, mixed)
