@@ -108,9 +108,11 @@ struct AxisDesc {
   // half-length DCT-II / III and DST-II / III stages (n = dtt_len).  DCT-IV /
   // DST-IV: of even dtt_len, an n = dtt_len / 2
   // point DFT of single lines, exp(-i pi (4j+1) / (4 dtt_len)), j < n, then
-  // exp(-i pi k / dtt_len), k < n; of odd dtt_len, a DFT of 2 dtt_len points of
-  // line pairs, exp(-i pi j / (2 dtt_len)), then exp(-i pi (2k+1) / (4 dtt_len))
+  // exp(-i pi k / dtt_len), k < n; of odd dtt_len, a DFT of dtt_len points of line
+  // pairs, the k-th output's signs of the real and imaginary part of frequency
+  // dtt_q0 + k dtt_q1 mod dtt_len
   const void *dtw;
+  int dtt_q0, dtt_q1;
   // Stages of the mixed kernels (any length): threads that share a tile
   // column, block size and LDS bytes of a launch.
   int rows, nthreads, lds_bytes;

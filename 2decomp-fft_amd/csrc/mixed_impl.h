@@ -102,7 +102,31 @@ __device__ __forceinline__ void est_divmod(int w, int n, float inv, int &q, int 
   }
 }
 
-template <typename T, int IO, bool LINES, int CLS, bool PK>
+// (a + b + c + d) sqrt(1/2), rounded once: the split of an odd DCT-IV, whose four
+// roundings would make it less accurate than the general kernel's longer DFT
+// (27 points in FP32 9.7e-8 there, 1.00e-7 with them).
+template <typename T>
+__device__ __forceinline__ T sum4_sqrt_half(T a, T b, T c, T d) {
+  constexpr double h = kRootCos[kRootOff[8] + 1];
+  if constexpr (sizeof(T) == 4) {
+    return (T)((((double)a + (double)b) + ((double)c + (double)d)) * h);
+  } else {
+    T err = T(0);
+    auto sum = [&](T x, T y) __attribute__((always_inline)) {  // Knuth's two-sum
+      const T s = x + y, v = s - x;
+      err += (x - (s - v)) + (y - v);
+      return s;
+    };
+    const T s = sum(sum(a, b), sum(c, d));
+    constexpr double l = -4.833646656726457e-17;
+    return s * h + (s * l + err * h);
+  }
+}
+
+// VAR = 1: c2c columns in the packed order of an exchange; real-to-real stages of
+// types 4 and 8 of even length; 2: those of odd length (in one kernel with the others
+// they cost registers and scratch: FP32 columns of 300 points 202 -> 245 us).
+template <typename T, int IO, bool LINES, int CLS, int VAR>
 __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out, int conj,
                                            long long tile) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -113,10 +137,11 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
   // real-to-real stages: the transform, and which of its ends are not the
   // points of the DFT themselves (types 3 and 7 merge the line into a Hermitian
   // sequence first, 2, 6 and odd-length 4, 8 split the result afterwards);
-  // types 4 and 8 of even length take one real line per tile column
+  // types 4 and 8 of even length take one real line per tile column, those of odd
+  // length a DFT of as many points of signed permuted ones (odd48)
   const int type = R2R ? d->dtt : 0, Lr = R2R ? d->dtt_len : 0;
-  const bool t48 = type == 4 || type == 8, single = t48 && Lr % 2 == 0;
-  const bool pre = type == 3 || type == 7, post = type == 2 || type == 6 || (t48 && Lr % 2 != 0);
+  constexpr bool PK = VAR == 1 && !R2R, single = VAR == 1 && R2R, odd48 = VAR == 2;
+  const bool pre = VAR == 0 && (type == 3 || type == 7), post = odd48 || (VAR == 0 && (type == 2 || type == 6));
   const bool alt = type >= 6;  // 6, 7, 8: signs (-1)^j
   const bool PAIRED = IO == IO_R2C || IO == IO_C2R || (R2R && !single);
   constexpr bool CHIRP = CLS == 2;
@@ -162,10 +187,10 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     const int nb = m / R;
     const long long step = (long long)nb * sji;
     if constexpr (R2R) {
-      // point J of the sequence that the DFT takes, types 1, 2, 4, 5, 6, 8: +- x_src
-      // (zero where src is no point of the line), src piecewise linear in J:
+      // point J of the sequence that the DFT takes, types 1, 2, even 4, 5, 6, even 8:
+      // +- x_src (zero where src is no point of the line), src piecewise linear in J:
       //   2, 6  x_0 x_2 x_4 ... x_5 x_3 x_1       1  e[j] = e[n-j] = x_j
-      //   5     e[j+1] = -e[n-j-1] = x_j          odd 4, 8  x_j, then zeros
+      //   5     e[j+1] = -e[n-j-1] = x_j
       // and (x_2J, x_{L-1-2J}) for even 4, 8.  All loads first, then the signs.
       const int h = (type == 2 || type == 6) ? (n + 1) / 2 : type == 1 ? Lr : type == 5 ? Lr + 1 : n;
       const int a1 = (type == 2 || type == 6 || single) ? 2 : 1, b1 = type == 5 ? -1 : 0;
@@ -181,6 +206,35 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
             const int j = src(b + s * nb);
             return in_base + (long long)((unsigned)j < (unsigned)Lr ? j : 0) * sji;
           };
+          if (odd48) {
+            // J = 2j + 1 mod L for one j.  With r = 2j + 1 in [0, 2L), the residue of r
+            // mod 8 decides between x_j and x_{L-1-j} and the sign (get_dtt4_odd_table)
+            auto at = [&](int s, bool &neg) __attribute__((always_inline)) {
+              const int J = b + s * nb, r = J & 1 ? J : J + n;
+              const int j = r & 2 ? n - 1 - (r >> 1) : r >> 1;
+              neg = (((r >> 2) ^ ((r & n) >> 1) ^ (alt ? j : 0)) & 1) != 0;
+              return !CHIRP || J < n ? j : -1;
+            };
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              bool neg;
+              const int j = at(s, neg);
+              const long long o = in_base + (long long)(j < 0 ? 0 : j) * sji;
+              if (adj_in && full) {
+                v[q * R + s] = gload_pair<T>(in, o);
+              } else {
+                v[q * R + s].x = gload_r<T>(in, o);
+                v[q * R + s].y = two ? gload_r<T>(in, o + d->in_s0) : T(0);
+              }
+            }
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              bool neg;
+              if (at(s, neg) < 0) v[q * R + s] = cpx<T>{T(0), T(0)};
+              else if (neg) v[q * R + s] = cpx<T>{-v[q * R + s].x, -v[q * R + s].y};
+            }
+            continue;
+          }
           if (single) {
 #pragma unroll
             for (int s = 0; s < R; ++s) {
@@ -212,15 +266,15 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
             for (int s = 0; s < R; ++s)
               if (b + s * nb >= h) v[q * R + s] = cpx<T>{-v[q * R + s].x, -v[q * R + s].y};
           }
-          if (CHIRP || type == 5 || (t48 && !single)) {
+          if (CHIRP || type == 5) {
 #pragma unroll
             for (int s = 0; s < R; ++s)
               if ((unsigned)src(b + s * nb) >= (unsigned)Lr) v[q * R + s] = cpx<T>{T(0), T(0)};
           }
-          if (t48) {  // exp(-i pi (4J+1) / 4L) of even L, exp(-i pi J / 2L) of odd L
+          if (single) {  // exp(-i pi (4J+1) / 4L)
 #pragma unroll
             for (int s = 0; s < R; ++s)
-              if (b + s * nb < (single ? n : Lr)) v[q * R + s] = cmul(v[q * R + s], gload<T>(d->dtw, b + s * nb));
+              if (b + s * nb < n) v[q * R + s] = cmul(v[q * R + s], gload<T>(d->dtw, b + s * nb));
           }
         }
       }
@@ -720,8 +774,8 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
     if (post) {
       // Z in LDS.  Types 2, 6: Y_k = 2 Re(w_q V_q) of each line of the pair, V
       // split from Z as in a real-to-complex transform, q = k (DCT-II) or
-      // L-1-k (DST-II).  Types 4, 8 of odd L (n = 2L): zeta_k = exp(-i pi (2k+1)
-      // / 4L) Z_k, Y_a = Re(zeta_k - zeta_{n-1-k}), Y_b the imaginary parts
+      // L-1-k (DST-II).  Types 4, 8 of odd L: the same with q = (2k+1) / 8 mod L and
+      // w_k = (+-1 -+ i) / sqrt 2, the signs from the table
       const int total = TX * Lr;
       const float inv_L = 1.0f / (float)Lr;
       for (int w = tid; w < total; w += nthr) {
@@ -734,18 +788,18 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
         }
         const long long cc = 2 * (c0b + tt);
         if (cc < d->C0r) {
-          const int q = alt ? Lr - 1 - k : k;
-          cpx<T> y;
-          if (t48) {
-            const cpx<T> cw = gload<T>(d->dtw, Lr + q);
-            const cpx<T> z1 = cmul(cw, lds[A(q, tt)]), z2 = cmul(cconj(cw), lds[A(n - 1 - q, tt)]);
-            y = cadd(z1, z2);
-          } else {
-            const cpx<T> zk = lds[A(q, tt)], zm = lds[A(q == 0 ? 0 : n - q, tt)];
-            const cpx<T> cs = gload<T>(d->dtw, q);
-            y = cpx<T>{cs.x * (zk.x + zm.x) + cs.y * (zk.y - zm.y),
-                       cs.x * (zk.y + zm.y) + cs.y * (zm.x - zk.x)};
+          const int kk = alt ? Lr - 1 - k : k;
+          int q = kk;
+          if (odd48) {
+            int turns;
+            est_divmod(d->dtt_q0 + kk * d->dtt_q1, Lr, inv_L, turns, q);
           }
+          const cpx<T> zk = lds[A(q, tt)], zm = lds[A(q == 0 ? 0 : n - q, tt)];
+          const cpx<T> cs = gload<T>(d->dtw, kk);
+          const cpx<T> y = odd48 ? cpx<T>{sum4_sqrt_half(cs.x * zk.x, cs.x * zm.x, cs.y * zk.y, -cs.y * zm.y),
+                                          sum4_sqrt_half(cs.x * zk.y, cs.x * zm.y, cs.y * zm.x, -cs.y * zk.x)}
+                                 : cpx<T>{cs.x * (zk.x + zm.x) + cs.y * (zk.y - zm.y),
+                                          cs.x * (zk.y + zm.y) + cs.y * (zm.x - zk.x)};
           const long long o = cc * d->out_s0 + c1 * d->out_s1 + (f0 + k) * sjo;
           if (cc + 1 < d->C0r && adj_out) {
             gstore_pair<T>(out, o, y);
@@ -789,14 +843,15 @@ __device__ __forceinline__ void mixed_tile(DescPtr d, const void *in, void *out,
 // room for.
 constexpr int mx_threads(int cls) { return cls == 1 ? 512 : 1024; }
 template <typename T>
-constexpr int mx_wpe(int cls) {
+constexpr int mx_wpe(int cls, int io) {
+  if (io == IO_R2R && cls == 1 && sizeof(T) == 8) return 3;  // (143-point DCT-I lines 580 -> 415 us)
   return cls != 1 ? (sizeof(T) == 8 ? 4 : 6) : (sizeof(T) == 8 ? 2 : 4);
 }
 
 // One grid (ng = 0: the stage of the arguments), or the tiles of several
 // grids (the same code, so that a batch's results equal the plans' own).
-template <typename T, int IO, bool LINES, int CLS, bool PK>
-__global__ void __launch_bounds__(mx_threads(CLS)) __attribute__((amdgpu_waves_per_eu(mx_wpe<T>(CLS))))
+template <typename T, int IO, bool LINES, int CLS, int VAR>
+__global__ void __launch_bounds__(mx_threads(CLS)) __attribute__((amdgpu_waves_per_eu(mx_wpe<T>(CLS, IO))))
     mixed_kernel(const AxisDesc *__restrict__ d, const void *in, void *out, int conj,
                  const MultiGroup *__restrict__ g, int ng, long long tiles) {
   long long it = xcd_tile((long long)blockIdx.x + (long long)blockIdx.y * gridDim.x, tiles);
@@ -809,10 +864,10 @@ __global__ void __launch_bounds__(mx_threads(CLS)) __attribute__((amdgpu_waves_p
     conj = g[gi].conj;
     it -= g[gi].tile0;
   }
-  mixed_tile<T, IO, LINES, CLS, PK>(desc_ptr(d), in, out, conj, it);
+  mixed_tile<T, IO, LINES, CLS, VAR>(desc_ptr(d), in, out, conj, it);
 }
 
-template <typename T, int IO, bool LINES, int CLS, bool PK>
+template <typename T, int IO, bool LINES, int CLS, int VAR>
 int mixed_go(const AxisDesc *dd, const AxisIo &io, const MultiGroup *g, int ng, long long tiles, int nt,
              size_t lds, hipStream_t st) {
   const long long nb = xcd_grid(tiles);
@@ -820,7 +875,7 @@ int mixed_go(const AxisDesc *dd, const AxisIo &io, const MultiGroup *g, int ng, 
   const long long gx = nb < (1LL << 20) ? nb : (1LL << 20);
   const long long gy = (nb + gx - 1) / gx;
   if (gy > 65535) return set_error(D2DHIP_ERR_UNSUPPORTED, "axis stage has too many tiles");
-  hipLaunchKernelGGL((mixed_kernel<T, IO, LINES, CLS, PK>), dim3((unsigned)gx, (unsigned)gy), dim3(nt), lds,
+  hipLaunchKernelGGL((mixed_kernel<T, IO, LINES, CLS, VAR>), dim3((unsigned)gx, (unsigned)gy), dim3(nt), lds,
                      st, dd, io.in, io.out, io.conj, g, ng, tiles);
   return hip_check(hipGetLastError(), "mixed_kernel launch");
 }
@@ -828,16 +883,23 @@ int mixed_go(const AxisDesc *dd, const AxisIo &io, const MultiGroup *g, int ng, 
 template <typename T, int IO, bool LINES, int CLS>
 int mixed_launch(const AxisDesc *dd, const AxisDesc &h, const AxisIo &io, hipStream_t st) {
   const long long tiles = (long long)h.tiles0 * h.C1;
+  auto go = [&](auto var) {
+    return mixed_go<T, IO, LINES, CLS, decltype(var)::value>(dd, io, nullptr, 0, tiles, h.nthreads, h.lds_bytes, st);
+  };
   if constexpr (IO == IO_C2C && !LINES) {
-    if (h.packj) return mixed_go<T, IO, LINES, CLS, true>(dd, io, nullptr, 0, tiles, h.nthreads, h.lds_bytes, st);
+    if (h.packj) return go(std::integral_constant<int, 1>{});
   }
-  return mixed_go<T, IO, LINES, CLS, false>(dd, io, nullptr, 0, tiles, h.nthreads, h.lds_bytes, st);
+  if constexpr (IO == IO_R2R) {
+    if (h.dtt == 4 || h.dtt == 8)
+      return h.dtt_len % 2 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
+  }
+  return go(std::integral_constant<int, 0>{});
 }
 
 template <typename T, int IO, bool LINES, int CLS>
 int mixed_launch_multi(const MultiGroup *g, int ng, long long tiles, int nt, size_t lds, hipStream_t st) {
   const AxisIo io = {nullptr, nullptr, 0};
-  return mixed_go<T, IO, LINES, CLS, false>(nullptr, io, g, ng, tiles, nt, lds, st);
+  return mixed_go<T, IO, LINES, CLS, 0>(nullptr, io, g, ng, tiles, nt, lds, st);
 }
 
 constexpr int kMaxLds = 160 * 1024;
@@ -851,13 +913,14 @@ hipError_t mixed_prepare() {
   if (e != hipSuccess) return e;
   const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
   if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
-  e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, false>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
-  if constexpr (IO == IO_C2C && !LINES) {
+  auto raise = [&](auto var) {
     if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, true>,
+      e = hipFuncSetAttribute((const void *)mixed_kernel<T, IO, LINES, CLS, decltype(var)::value>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
-  }
+  };
+  raise(std::integral_constant<int, 0>{});
+  if constexpr ((IO == IO_C2C && !LINES) || IO == IO_R2R) raise(std::integral_constant<int, 1>{});
+  if constexpr (IO == IO_R2R) raise(std::integral_constant<int, 2>{});
   if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
   return e;
 }

@@ -485,15 +485,16 @@ int get_bluestein(d2dhip_plan_s *p, int n, int M, const std::vector<int> &order,
 }
 
 int get_dtt4_twiddles(d2dhip_plan_s *p, int L, const void **out);
-int get_dtt4_odd_twiddles(d2dhip_plan_s *p, int L, const void **out);
+int get_dtt4_odd_table(d2dhip_plan_s *p, int L, const void **out);
+int inverse_of_8(int L);
 
 // Points of the DFT that the kernels of any length run a stage through: the
 // line's, or for a real-to-real stage its length L (types 2, 3, 6, 7), the
 // extension's (2(L-1), 2(L+1) for types 1, 5), or for types 4, 8 half of an even
-// L and twice an odd one.
+// L and an odd one itself.
 int stage_dft(const StageGeom &g) {
   if (g.io != IO_R2R) return g.n;
-  if (g.dtt == 4 || g.dtt == 8) return g.dtt_len % 2 ? 2 * g.dtt_len : g.dtt_len / 2;
+  if (g.dtt == 4 || g.dtt == 8) return g.dtt_len % 2 ? g.dtt_len : g.dtt_len / 2;
   return g.n;
 }
 
@@ -536,9 +537,13 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
       return set_error(D2DHIP_ERR_UNSUPPORTED, "mixed kernel: length not covered");
     const int M = mixed_length(*fv, line);
     if (M != line && (st = get_bluestein(p, line, M, radices, &bt))) return st;
-    if (t48 && (st = g.dtt_len % 2 ? get_dtt4_odd_twiddles(p, g.dtt_len, &dtw)
+    if (t48 && (st = g.dtt_len % 2 ? get_dtt4_odd_table(p, g.dtt_len, &dtw)
                                    : get_dtt4_twiddles(p, g.dtt_len, &dtw)))
       return st;
+    if (t48 && g.dtt_len % 2) {
+      a.dtt_q0 = inverse_of_8(g.dtt_len);
+      a.dtt_q1 = 2 * a.dtt_q0 % g.dtt_len;
+    }
   } else if (fv) {
     radices = fv->radices;
     if (fv->io == IO_DTT4 && (st = get_dtt4_twiddles(p, g.dtt_len, &dtw))) return st;
@@ -784,33 +789,51 @@ int get_dtt4_twiddles(d2dhip_plan_s *p, int L, const void **out) {
   return hip_check(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice), "hipMemcpy");
 }
 
-// exp(-i pi j / (2L)), j < L, then exp(-i pi (2k+1) / (4L)), k < L: the pre- and
-// post-twiddles of DCT-IV / DST-IV of odd L through a DFT of 2L points (kept
-// under key -L, which only odd lengths use for it).
-int get_dtt4_odd_twiddles(d2dhip_plan_s *p, int L, const void **out) {
+int inverse_of_8(int L) {  // mod L, odd
+  int b = 0;
+  while (8 * b % L != 1 % L) ++b;
+  return b;
+}
+
+// DCT-IV of odd L without multiplications by angles.  With m = (2j+1)(2k+1),
+// a = 1/L mod 8 and b = 1/8 mod L, m / 8L = a m / 8 + b m / L up to whole turns, so
+//   X_k = 2 sum_j x_j cos(2 pi m / 8L)
+//       = sqrt 2 sum_j x_j [c(a m) cos(2 pi b m / L) - s(a m) sin(2 pi b m / L)],
+// where c and s (the signs of the cosine and sine of an odd multiple of pi/4) are
+// the characters +--+ and ++-- of 1, 3, 5, 7 mod 8, hence products of one factor
+// in j and one in k.  The cosine sum sees the part of a sequence even in p = 2j+1
+// mod L, the sine sum the odd part: both are parts of the signed permutation z_p
+// that the kernels load (z_p = x_j for r = 2j+1 = 1 mod 8, -x_j for 5, and for 3
+// and 7 +-x_{L-1-j}, + - for L = 1 mod 4, - + for 3), and with its DFT F at q =
+// b (2k+1) mod L
+//   X_k = sqrt 2 [c(a) c(2k+1) Re F_q + s(a) s(2k+1) Im F_q].
+// The table holds the two signs of every k, under key -L, which only odd lengths
+// use for it.  (Through 2L points with twiddles before and after, FP64 errors were
+// up to 19 % above the general kernel's through 8L; now they are below it, and the
+// DFT is half as long.)
+int get_dtt4_odd_table(d2dhip_plan_s *p, int L, const void **out) {
   auto it = p->dtw.find(-L);
   if (it != p->dtw.end()) {
     *out = it->second;
     return D2DHIP_SUCCESS;
   }
   const int rb = p->rb;
-  std::vector<unsigned char> h((size_t)L * 4 * rb);
-  for (int k = 0; k < 2 * L; ++k) {
-    long double c, s;
-    if (k < L)
-      unit_root(k, 4LL * L, c, s);
-    else
-      unit_root(2LL * (k - L) + 1, 8LL * L, c, s);
+  std::vector<unsigned char> h((size_t)L * 2 * rb);
+  auto c = [](int r) { return r % 8 == 1 || r % 8 == 7 ? 1 : -1; };
+  auto s = [](int r) { return r % 8 == 1 || r % 8 == 3 ? 1 : -1; };
+  for (int k = 0; k < L; ++k) {
+    // (L is its own inverse mod 8)
+    const int re = c(L) * c(2 * k + 1), im = s(L) * s(2 * k + 1);
     if (rb == 8) {
-      reinterpret_cast<double *>(h.data())[2 * k] = (double)c;
-      reinterpret_cast<double *>(h.data())[2 * k + 1] = (double)-s;
+      reinterpret_cast<double *>(h.data())[2 * k] = re;
+      reinterpret_cast<double *>(h.data())[2 * k + 1] = im;
     } else {
-      reinterpret_cast<float *>(h.data())[2 * k] = (float)c;
-      reinterpret_cast<float *>(h.data())[2 * k + 1] = (float)-s;
+      reinterpret_cast<float *>(h.data())[2 * k] = (float)re;
+      reinterpret_cast<float *>(h.data())[2 * k + 1] = (float)im;
     }
   }
   void *d = nullptr;
-  if (hipMalloc(&d, h.size()) != hipSuccess) return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(DTT twiddles)");
+  if (hipMalloc(&d, h.size()) != hipSuccess) return set_error(D2DHIP_ERR_ALLOC, "hipMalloc(DTT table)");
   p->dtw[-L] = d;
   *out = d;
   return hip_check(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice), "hipMemcpy");
@@ -2048,8 +2071,7 @@ long long d2dhip_plan_device_bytes(d2dhip_plan p) {
   if (!p) return 0;
   long long b = (long long)p->wk_bytes;
   for (auto &kv : p->tw) b += (long long)kv.second.bytes;
-  for (auto &kv : p->dtw)  // (odd lengths under a negative key: two entries a point)
-    b += (long long)std::abs(kv.first) * (kv.first < 0 && kv.first % 2 ? 4 : 2) * p->rb;
+  for (auto &kv : p->dtw) b += (long long)std::abs(kv.first) * 2 * p->rb;
   return b;
 }
 

@@ -113,3 +113,13 @@ def test_real_to_real_smooth_lengths(d2d, torch_gpu, t, points, axis, prec):
 def test_real_to_real_bluestein_lengths(d2d, torch_gpu, t, points, axis, prec):
     general, mixed = _dtt_errors(d2d, torch_gpu, t, points, axis, prec)
     assert mixed < BOUND * general, (general, mixed)
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("points", [17, 23, 27, 49, 63, 99, 149, 243, 255, 299, 405, 32, 64, 100, 254, 300, 382, 486, 512])
+@pytest.mark.parametrize("t", [4, 8])
+def test_dct4(d2d, torch_gpu, t, points, axis, prec):
+    """Odd lengths through a DFT of as many points, even ones of half as many."""
+    general, mixed = _dtt_errors(d2d, torch_gpu, t, points, axis, prec)
+    assert mixed < BOUND * general, (general, mixed)
