@@ -22,9 +22,9 @@
 
 namespace d2dhip {
 
-struct alignas(16) H16 {
-  unsigned long long a, b;
-};
+// (a vector, not a struct: arrays of a struct went to scratch memory, 80 bytes a
+// lane)
+using H16 = unsigned long long __attribute__((ext_vector_type(2)));
 
 // 16 bytes of adjacent cells, aligned as one cell is.
 template <typename E>
@@ -48,20 +48,24 @@ struct HaloArgs {
 // the pencil gives the cell that the axis-by-axis exchange would have copied:
 // a cell of the pencil, or, where the other axis is not periodic and the cell
 // lies in its halo, a cell of the array that nothing writes.  2^lg threads
-// share a row (i fastest), 16 bytes each, two loads ahead of their stores.
+// share a row (i fastest): 16 bytes of the pencil's part each, two loads (of whole
+// 16-byte cells: one) ahead of their stores, and one cell of the two ends, loaded with
+// them; so a row that the threads fill takes one round whatever its ends.
 //
-// Bound by HBM: 512^3 FP64, level 2, x-pencil 366 -> 346 us (6.4 TB/s of cells
-// read and written once), y-pencil 403 -> 374, FP32 z-pencil 310 -> 208, against
-// a copy of the pencil by rows and a launch per filled axis.  Small arrays are
-// bound by the launch (64^3 14.1 -> 8.2 us), short rows by the lanes that a
-// block per row left idle (27 x 700 x 600 176 -> 45 us).
+// Bound by HBM, against a copy of the pencil by rows and a launch per filled axis,
+// all axes periodic, level 2, 512^3: FP64 x-pencil 366 -> 343 us (6.4 TB/s of cells
+// read and written once), y-pencil 403 -> 344, FP32 z-pencil 311 -> 176; complex FP64
+// 256^3 y-pencil 100 -> 88.  Small arrays are bound by the launch (64^3 13.7 -> 8.4 us),
+// short rows by the lanes that a block per row left idle (27 x 700 x 600 152 -> 24
+// us).  Without periodic axes there is one copy on either side: level with it but for
+// complex FP64, which is 2 to 6 % slower on rows that leave threads idle.
 template <typename E>
 __global__ void __launch_bounds__(256) halo_update_kernel(const E *__restrict__ in, E *arr, HaloArgs a,
                                                           int lg) {
   using Q = typename Cells<E>::Q;
-  constexpr int V = Cells<E>::V, U = 2;
-  const int lane = threadIdx.x & ((1 << lg) - 1), n1 = a.n[0], s1 = a.s[0], o1 = a.o[0];
-  const int nv = (n1 + V - 1) / V;
+  constexpr int V = Cells<E>::V, U = V == 1 ? 1 : 2;
+  const int lanes = 1 << lg, lane = threadIdx.x & (lanes - 1), n1 = a.n[0], s1 = a.s[0], o1 = a.o[0];
+  const int nv = s1 / V, ne = n1 - s1;
   const long long rows = (long long)a.n[1] * a.n[2], step = (long long)gridDim.x * (256 >> lg);
   for (long long row = (long long)blockIdx.x * (256 >> lg) + (threadIdx.x >> lg); row < rows; row += step) {
     const int k = rows >> 31 ? (int)(row / a.n[1]) : (int)((unsigned)row / (unsigned)a.n[1]);
@@ -78,49 +82,36 @@ __global__ void __launch_bounds__(256) halo_update_kernel(const E *__restrict__ 
         open = true;
       }
     }
-    // cell i of the source row is arow[i] or, within the pencil, src[i]
+    // cell i of the source row is arow[i] or, within the pencil, src[i - o1]
     const E *arow = arr + ((long long)(c[1] + a.o[2]) * a.n[1] + c[0] + a.o[1]) * n1;
-    const E *src = open ? arow : in + ((long long)c[1] * a.s[1] + c[0]) * s1 - o1;
+    const E *src = open ? arow + o1 : in + ((long long)c[1] * a.s[1] + c[0]) * s1;
     E *dst = arr + row * n1;
     const bool copy = moved || !open;
-    // where cell i of the row comes from, if it is written
-    auto source = [&](int i) -> const E * {
-      const int q = i - o1;
-      if (i >= n1) return nullptr;
-      if (q >= 0 && q < s1) return copy ? src + i : nullptr;
-      if (a.w[0]) return src + (q < 0 ? i + s1 : i - s1);
-      return moved ? arow + i : nullptr;
+    // end cell e (those below the pencil's part, then those above) and where it
+    // comes from, if it is written
+    auto end_source = [&](int e) -> const E * {
+      if (e >= ne) return nullptr;
+      if (a.w[0]) return src + (e < o1 ? e + s1 - o1 : e - o1);
+      return moved ? arow + (e < o1 ? e : e + s1) : nullptr;
     };
-    for (int b = lane; b < nv; b += U << lg) {
-      Q v[U];
-      E e[U][V];
-      int kind[U];  // 2: V cells of the pencil, 1: the ends of a row, cell by cell
+    const E *from = end_source(lane);
+    E end{};
+    if (from) end = *from;
+    if (copy) {
+      for (int b = lane; b < nv; b += U * lanes) {
+        Q v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i0 = (b + (u << lg)) * V;
-        kind[u] = i0 >= n1 ? 0 : (i0 >= o1 && i0 + V <= o1 + s1) ? (copy ? 2 : 0) : 1;
-        if (kind[u] == 2) {
-          v[u] = *reinterpret_cast<const Q *>(src + i0);
-        } else if (kind[u] == 1) {
+        for (int u = 0; u < U; ++u)
+          if (b + u * lanes < nv) v[u] = *reinterpret_cast<const Q *>(src + (b + u * lanes) * V);
 #pragma unroll
-          for (int t = 0; t < V; ++t) {
-            const E *from = source(i0 + t);
-            if (from) e[u][t] = *from;
-          }
-        }
+        for (int u = 0; u < U; ++u)
+          if (b + u * lanes < nv) *reinterpret_cast<Q *>(dst + o1 + (b + u * lanes) * V) = v[u];
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i0 = (b + (u << lg)) * V;
-        if (kind[u] == 2) {
-          *reinterpret_cast<Q *>(dst + i0) = v[u];
-        } else if (kind[u] == 1) {
-#pragma unroll
-          for (int t = 0; t < V; ++t)
-            if (source(i0 + t)) dst[i0 + t] = e[u][t];
-        }
-      }
+      for (int i = nv * V + lane; i < s1; i += lanes) dst[o1 + i] = src[i];
     }
+    if (from) dst[lane < o1 ? lane : lane + s1] = end;
+    for (int e = lane + lanes; e < ne; e += lanes)
+      if (const E *f = end_source(e)) dst[e < o1 ? e : e + s1] = *f;
   }
 }
 
@@ -170,11 +161,11 @@ static int halo_run(const void *in, void *arr, const int s[3], const int n[3], c
     }
     for (int q = 0; q < 2; ++q) a.w[order[q]] = wrap[q];
     // The power of two of threads to a row that fills them best: as many as the
-    // row has 16-byte groups, or half of that where the last pass would be less
-    // than an eighth full.  us with 256 / 128 / 64 / 32 threads, level 2: FP64 rows
-    // of 512 cells 346 / 370 / 388 / 416, of 516 392 / 370 / 440 / 474; FP32 rows of
-    // 516 340 / 242 / 210 / 230, of 156 - / - / 56 / 46.
-    const int nv = (n[0] + Cells<E>::V - 1) / Cells<E>::V;
+    // pencil's row has 16-byte groups, or half of that where the last round would be
+    // less than an eighth full.  us with 256 / 128 / 64 / 32 threads, level 2: FP64
+    // rows of 512 cells 344 / 381 / 380 / 402, FP32 ones 216 / 171 / 191 / 189, of 150
+    // 102 / 56 / 35 / 24; complex FP64 rows of 150 132 / 112 / 117 / 133.
+    const int nv = (s[0] + Cells<E>::V - 1) / Cells<E>::V;
     int lg = 0;
     while (lg < 8 && (2LL << lg) <= nv) ++lg;
     if (lg && (nv - 1) % (1 << lg) + 1 <= (1 << lg) / 8) --lg;
