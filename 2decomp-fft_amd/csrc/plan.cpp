@@ -614,10 +614,27 @@ int configure(d2dhip_plan_s *p, int idx, int c) {
   return D2DHIP_SUCCESS;
 }
 
+// Whether a batch runs this stage on the persistent tile of its length: the c2c
+// stages of whole grids whose three lengths have one.
+bool batch_stage(const d2dhip_plan_s *p, int idx) {
+  if (idx > 2 || p->multi) return false;
+  const int n[3] = {p->nx, p->ny, p->nz};
+  for (int a = 0; a < 3; ++a) {
+    bool found = false;
+    for (const PersistKind &k : persist_kinds(p->rb)) found = found || (k.n == n[a] && k.lines == (a == 0 ? 1 : 0));
+    if (!found) return false;
+  }
+  return true;
+}
+
 // Candidates that run only where a caller chooses them: convolutions shorter
-// than the general kernel's, which are less accurate.
-bool only_chosen(const StageGeom &g, int c) {
-  return c >= 0 && g.cands[c]->mixed && mixed_short(*g.cands[c], stage_dft(g));
+// than the general kernel's, which are less accurate, and any-length kernels in
+// the stages of a persistent batch, whose other radices would set the plan's own
+// result apart from the batch's in the last bits (256^3 FP64 c2c: 4 % of a stage's
+// time given up for that).
+bool only_chosen(const d2dhip_plan_s *p, int idx, int c) {
+  const StageGeom &g = p->geom[idx];
+  return c >= 0 && g.cands[c]->mixed && (mixed_short(*g.cands[c], stage_dft(g)) || batch_stage(p, idx));
 }
 
 // The same for a real-to-real stage with a compiled tile (its first candidate)
@@ -669,8 +686,9 @@ int dtt_choice(const d2dhip_plan_s *p, const StageGeom &g) {
 // points 3.7 against 4.1), other real columns on the first tile that leaves
 // room for a second workgroup on the CU (c2r columns of 1152 points 3.5 on 8
 // columns, 4.3 on 4).
-int default_choice(const d2dhip_plan_s *p, const StageGeom &g) {
-  if (g.cands.empty() || only_chosen(g, 0)) return -1;
+int default_choice(const d2dhip_plan_s *p, int idx) {
+  const StageGeom &g = p->geom[idx];
+  if (g.cands.empty() || only_chosen(p, idx, 0)) return -1;
   if (g.cands[0]->mixed || g.cands[0]->mf) return 0;
   if (g.io == IO_R2R) return dtt_choice(p, g);
   const bool f64 = p->rb == 8, lines = g.axis == 0, real = g.io != IO_C2C;
@@ -679,7 +697,7 @@ int default_choice(const d2dhip_plan_s *p, const StageGeom &g) {
   const bool cached = g.out_elems * (g.io == IO_C2R ? 1 : 2) * p->rb < (128ll << 20);
   const bool any = (g.n <= n_short && !cached) || (g.io == IO_R2C && !lines && g.n >= 896);
   for (size_t c = 0; c < g.cands.size(); ++c)
-    if (any && g.cands[c]->mixed) return (int)c;
+    if (any && g.cands[c]->mixed && !only_chosen(p, idx, (int)c)) return (int)c;
   if (real && !lines)
     for (size_t c = 0; c < g.cands.size(); ++c)
       if (!g.cands[c]->mixed && g.cands[c]->lds_bytes <= 80 * 1024) return (int)c;
@@ -726,7 +744,7 @@ int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, 
     const int st = general_fits(p, g);
     if (st) return st;
   }
-  return configure(p, idx, default_choice(p, g));
+  return configure(p, idx, default_choice(p, idx));
 }
 
 // (cos, sin)(pi k / (2L)), k < L, in long double rounded to the plan's
@@ -897,7 +915,7 @@ int make_dtt_stage(d2dhip_plan_s *p, int idx, int axis, int type, int first, int
     const int st = general_fits(p, g);
     if (st) return st;
   }
-  return configure(p, idx, default_choice(p, g));
+  return configure(p, idx, default_choice(p, idx));
 }
 
 int upload_chunk_descs(d2dhip_plan_s *p);
@@ -1157,7 +1175,7 @@ int tune_stages(d2dhip_plan_s *p) {
       int c = -1;
       for (size_t k = 0; k < g.cands.size(); ++k)
         if (it->second == g.cands[k]->name) c = (int)k;
-      if ((c >= 0 && !only_chosen(g, c)) || it->second == "general") {
+      if ((c >= 0 && !only_chosen(p, i, c)) || it->second == "general") {
         st = configure(p, i, c);
         continue;
       }
@@ -1194,7 +1212,7 @@ int tune_stages(d2dhip_plan_s *p) {
     const int nc = (int)g.cands.size();
     std::vector<float> t(nc + 1, 1e30f);  // t[c + 1]: candidate c, -1 = general
     for (int c = -1; c < nc && !st; ++c) {
-      if (only_chosen(g, c)) continue;
+      if (only_chosen(p, i, c)) continue;
       if (configure(p, i, c)) continue;  // e.g. the general kernel cannot run this length
       st = measure(c, &t[c + 1]);
     }

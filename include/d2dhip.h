@@ -366,8 +366,10 @@ int d2dhip_batch_set_stream(d2dhip_batch batch, void *stream);
  * persistent launch when every c2c stage of every plan has a length with a
  * persistent tile (32, 48, 64, 80, 96, 128, 160, 192, 256): its workgroups
  * run those specialised tiles (d2dhip_batch_persistent_tiles reports 1), and
- * results are bit-identical to the plans' calls on any specialised kernel of
- * each length.  Otherwise the default runs as D2DHIP_BATCH_GROUPED (one
+ * results are bit-identical to the plans' calls on any compiled tile of each
+ * length: the kernels that untuned plans of such grids run, and tuned ones
+ * choose from beside the general kernel (the any-length kernels, named "mixed",
+ * run there only when d2dhip_plan_set_stage_kernel chooses them).  Otherwise the default runs as D2DHIP_BATCH_GROUPED (one
  * persistent launch on general-kernel tiles is about 3x slower than the
  * plans' own kernels).  D2DHIP_BATCH_PERSISTENT_GENERAL forces the
  * persistent launch on the general kernel's tiles, bit-identical to the
