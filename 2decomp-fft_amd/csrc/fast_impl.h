@@ -754,6 +754,7 @@ static FastVariant make_variant(const char *name) {
   v.rb = (int)sizeof(T);
   v.io = IO;
   v.lines = LINES ? 1 : 0;
+  v.split = XM ? 1 : 0;
   v.n = N;
   v.TX = TX;
   v.NT = NT;

@@ -16,6 +16,7 @@ struct FastVariant {
   int mixed = 0;   // > 0: any length (mixed_impl.h); shape and radices from mixed_shape
   int io = 0;      // IO_C2C / IO_R2C / IO_C2R
   int lines = 0;   // 1: contiguous lines (x axis), 0: strided columns
+  int split = 0;   // 1: the exchanges take real and imaginary parts apart (XM 1, 2)
   int n = 0;       // FFT length
   int TX = 1, NT = 64;
   size_t lds_bytes = 0;

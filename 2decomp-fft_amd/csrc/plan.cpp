@@ -645,8 +645,8 @@ bool only_chosen(const d2dhip_plan_s *p, int idx, int c) {
 //   273: the tile up to 128 MB.  FP32 columns of 1024 points 19 / 28, 505 / 641.
 //   DCT-IV columns of 512 points (half of the line's) FP64 14 / 17, 382 / 374,
 //   FP32 18 / 21, 488 / 449: the tile up to 128 MB, FP32 1024 points 20 / 31,
-//   566 / 708 at every size; lines of 64 points FP64 16 / 18 (40 / 40 at 60 MB),
-//   427 / 346: up to 32 MB.
+//   566 / 708 at every size, and 64 points 325 / 361; lines of 64 points FP64 16 /
+//   18 (40 / 40 at 60 MB), 427 / 346: up to 32 MB.
 //   DCT-I of 128-point extensions, 8 and 24 MB: FP64 lines 9 / 10, 20 / 19: the
 //   tile up to 16 MB; where its passes hold 8 values a lane (64 and 512 points)
 //   up to 128 MB (60 MB, 512 points: 35 / 38).  FP32 columns of 256 points 22 /
@@ -663,7 +663,7 @@ int dtt_choice(const d2dhip_plan_s *p, const StageGeom &g) {
   if (tile.io == IO_DTT2 || tile.io == IO_DTT3)
     keep = lines || !f64 || mb < 128;
   else if (tile.io == IO_DTT4)
-    keep = f32_1024 || mb < (lines ? 32 : 128);
+    keep = f32_1024 || (!f64 && !lines && tile.n == 64) || mb < (lines ? 32 : 128);
   else
     keep = f32_1024 || mb < 16 ||
            (mb < 128 && (f64 ? *std::max_element(tile.radices.begin(), tile.radices.end()) <= 8 : !lines));
@@ -671,37 +671,56 @@ int dtt_choice(const d2dhip_plan_s *p, const StageGeom &g) {
 }
 
 // Candidate that an untuned stage runs: the first registered tile of its
-// length, with two rules measured on 1.2 GB stages of every registered length
-// (TB/s, compiled tile / any-length kernel).
-// Short lengths of pencils that come from HBM run on the any-length kernels,
-// whose tiles are wider: FP64
-// columns of 64 / 128 / 256 points 4.6 / 4.6 / 4.7 against 5.3 / 5.2 / 5.1 (of 320
-// 4.7 against 4.6), FP32 of 192 / 256 points 3.4 / 4.8 against 5.0 / 5.1 (of 384
-// 4.6 against 4.2); c2r lines of 80 / 96 / 128 / 160 points 3.3 / 3.2 / 4.1 / 4.1
-// against 4.8 / 5.3 / 5.3 / 5.4 (of 192 5.5 against 5.4), r2c lines of 80 / 96
-// points 4.4 / 4.7 against 5.2 / 5.3 (of 128 5.4 against 4.9).  Pencils below
-// 128 MB stay in the memory-side cache, where the compiled tiles' shorter
-// latency counts more (128^3: 12.0 against 12.8 us a stage).
-// r2c columns of 896 points and more run there too (FP64 3.7 against 4.0, 1024
-// points 3.7 against 4.1), other real columns on the first tile that leaves
-// room for a second workgroup on the CU (c2r columns of 1152 points 3.5 on 8
-// columns, 4.3 on 4).
+// length, the fastest on pencils that come from HBM, with rules measured on
+// pencils of 24 to 600 MB of every registered length.  (us, compiled tile /
+// any-length kernel; the largest side of the stage in MB before the colon.)
+//
+// Pencils below 32 MB: tiles whose exchange takes real and imaginary parts apart
+// fit more workgroups on a CU, which such a pencil does not fill, and pay two more
+// barriers: the first tile with a plain exchange.  FP64 columns split / plain, 24:
+// of 1024 points 15.6 / 14.3, 1536 16.1 / 14.6, 2048 21 / 15 (48: 26 / 29); r2c lines
+// of 1600 points 17.7 / 15.6 (48: 26 / 28).
+//
+// Short lengths of pencils of 128 MB and more, which do not stay in the memory-side
+// cache, run on the any-length kernels, whose tiles are wider.  FP64 c2c columns of
+// 64 / 256 points 600: 345 / 242, 307 / 264 (of 320 299 / 301); 80: 26 / 26, 30 / 33.
+// FP64 real columns up to 192 points, from 256 MB up to 256 points: c2r of 256 200:
+// 104 / 105, 300: 134 / 158, r2c 130: 58 / 65, 600: 310 / 298.  FP32 ones up to 200
+// points: c2r of 192 130: 75 / 58, of 240 600: 257 / 278, r2c of 256 200: 93 / 104.
+// Lines: c2r of 80 / 96 / 128 points FP64 600: 395 / 265, 407 / 248, 313 / 244 (of
+// 192 227 / 236); r2c of 80 / 96 points FP64 288 / 245, 271 / 244 (of 128 236 / 257).
+//
+// r2c columns of 896 points and more, from 32 MB: FP64 of 896 to 1024 points (1000
+// points 80: 45 / 42, 600: 345 / 314; above, the tile: 1152 points 317 / 390, 2048
+// 393 / 421), and where a tile's lanes hold more than 20 values, which leaves few
+// waves: FP64 1536 points up to 512 MB (130: 93 / 83, 600: 416 / 445), FP32 1536
+// points 80: 55 / 42, 600: 444 / 426 (16 values: 1024 points 80: 42 / 46, 600: 359 /
+// 366).  Other real columns run on the first tile that leaves room for a second
+// workgroup on the CU (FP64 c2r columns of 640 points 8 / 4 columns, 24: 19 / 14).
 int default_choice(const d2dhip_plan_s *p, int idx) {
   const StageGeom &g = p->geom[idx];
   if (g.cands.empty() || only_chosen(p, idx, 0)) return -1;
   if (g.cands[0]->mixed || g.cands[0]->mf) return 0;
   if (g.io == IO_R2R) return dtt_choice(p, g);
   const bool f64 = p->rb == 8, lines = g.axis == 0, real = g.io != IO_C2C;
-  const int n_short = !lines ? (real ? 256 : f64 ? 300 : 256)
-                             : (g.io == IO_R2C ? (f64 ? 100 : 192) : 160);
-  const bool cached = g.out_elems * (g.io == IO_C2R ? 1 : 2) * p->rb < (128ll << 20);
-  const bool any = (g.n <= n_short && !cached) || (g.io == IO_R2C && !lines && g.n >= 896);
-  for (size_t c = 0; c < g.cands.size(); ++c)
-    if (any && g.cands[c]->mixed && !only_chosen(p, idx, (int)c)) return (int)c;
-  if (real && !lines)
-    for (size_t c = 0; c < g.cands.size(); ++c)
-      if (!g.cands[c]->mixed && g.cands[c]->lds_bytes <= 80 * 1024) return (int)c;
-  return 0;
+  const long long mb = (g.out_elems * (g.io == IO_C2R ? 1 : 2) * p->rb) >> 20;
+  int tile = -1, any = -1;
+  for (int c = (int)g.cands.size() - 1; c >= 0; --c) {
+    const FastVariant &v = *g.cands[c];
+    if (v.mixed) any = c;
+    else if (real && !lines ? v.lds_bytes <= 80 * 1024 : mb >= 32 || !v.split) tile = c;
+  }
+  if (tile < 0) tile = 0;
+  if (any < 0 || only_chosen(p, idx, any)) return tile;
+  const int n_short = lines ? (g.io == IO_R2C ? (f64 ? 100 : 192) : 160)
+                            : real ? (f64 ? (mb < 256 ? 192 : 256) : 200) : (f64 ? 300 : 256);
+  if (g.n <= n_short && mb >= 128) return any;
+  if (g.io == IO_R2C && !lines && g.n >= 896 && mb >= 32) {
+    const FastVariant &v = *g.cands[tile];
+    if (f64 && g.n <= 1024) return any;
+    if (v.n * v.TX / v.NT > 20 && (!f64 || mb < 512)) return any;
+  }
+  return tile;
 }
 
 int make_stage(d2dhip_plan_s *p, int idx, int axis, int io, const StageIo &sio, long long in_elems,

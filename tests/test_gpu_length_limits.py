@@ -115,3 +115,15 @@ def test_small_pencils_run_the_compiled_real_to_real_tiles(d2d, torch_gpu, prec)
             assert all("mixed" not in small[s] for s in (7, 8, 10, 11)), (n, t, small)
     large = d2d.FFTEngine(1, 257, 257, 3000, prec=prec, opt_DTT=(4, 4, 2)).dtt_stage_kernels()
     assert "mixed" in large[7] and "mixed" in large[8]
+
+
+def test_defaults_of_small_pencils(d2d, torch_gpu):
+    """Pencils below 32 MB start on tiles with a plain exchange, large ones on
+    those that take real and imaginary parts apart; r2c columns of 1152 points on
+    the compiled tile, of 1000 points on the any-length kernel from 32 MB."""
+    small = d2d.FFTEngine(1, 16, 1536, 16).stage_kernels()["c2c_y"]
+    large = d2d.FFTEngine(1, 32, 1536, 64).stage_kernels()["c2c_y"]
+    assert " xs" not in small and " xs" in large
+    for n, nx, mixed in ((1000, 16, False), (1000, 256, True), (1152, 256, False), (1152, 512, False)):
+        k = d2d.FFTEngine(3, nx, 32, n).stage_kernels()["r2c"]
+        assert ("mixed" in k) == mixed, (n, nx, k)
