@@ -5,16 +5,20 @@
 // pass, which costs it 248 VGPRs (2 waves per SIMD) and callee-saved
 // registers spilled around every call.  Here the radix of a pass is a
 // compile-time case of a uniform switch and everything else (length, tile,
-// rows) is read from the descriptor, so one kernel serves every length at
-// 4 waves per SIMD with no calls and no spills.
+// rows) is read from the descriptor, so one kernel serves every length
+// without calls.  In FP64 the lengths with factors 2-7 and the chirps hold up to
+// 128 VGPRs (4 waves per SIMD), factors up to 17 up to 183 (2-3 waves); FP32 58-109
+// (4-8 waves).  Only packed columns (60 bytes a lane in FP64, 52 in FP32), the FP64
+// real-to-real lines of factors up to 17 (36) and some of the chirps (8-68) use
+// scratch.
 //
 // A workgroup owns a tile of TX columns of n points; `rows` threads share a
-// column and take butterflies row, row + rows, ... of every pass, at most 16
-// values each.  Strided columns put consecutive threads on consecutive tile
-// columns (one run of 128 bytes or more per point); contiguous lines put
-// them on consecutive points of a line.  The first pass reads HBM, the last
-// writes HBM, those in between exchange through LDS; real transforms pair
-// two real columns as the general kernel does.
+// column and take butterflies row, row + rows, ... of every pass, about 10
+// values each (mx_nb; up to 20 in FP32 columns).  Strided columns put
+// consecutive threads on consecutive tile columns (one run of 128 bytes or more
+// per point); contiguous lines put them on consecutive points of a line.  The
+// first pass reads HBM, the last writes HBM, those in between exchange through
+// LDS; real transforms pair two real columns as the general kernel does.
 //
 // Measured against the general kernel on 0.8 GB stages, FP64 TB/s of the bytes
 // read and written once (columns c2c / lines r2c / lines c2r):
@@ -24,17 +28,20 @@
 // Class 2 ("chirp") runs lengths with a prime factor above 17 by Bluestein's
 // algorithm over a length m >= 2n - 1 (mixed_length), in place (the general kernel
 // sweeps the LDS tile twelve times at n = 382): columns of 101 / 191 / 382 / 1021
-// points 1.0 / 0.8 / 0.8 / 0.9 -> 2.4 / 2.1 / 1.9 / 1.8 TB/s.  It is bound by latency and the texture path: at n = 382 the
-// vector units are busy 40 % of the time, the twiddle, chirp and spectrum
-// loads keep the address unit busy half of it.  Radices end at 12, where
-// FP64 still fits 128 VGPRs with a pass's twiddles loaded ahead.
+// points 1.0 / 0.8 / 0.8 / 0.9 -> 2.4 / 2.1 / 1.9 / 1.8 TB/s.  It is bound by latency and
+// by the loads of twiddles, chirp and spectrum: on the 382-point columns of a
+// 450 x 405 grid waves wait 49 % of their time, the address units are busy 61 %
+// of the launch, the vector units half of the time that a workgroup is on the
+// CU.  Its radices are those of its convolution lengths, up to 12, where FP64 still
+// fits 128 VGPRs with a pass's twiddles loaded ahead.
 // Real-to-real stages (columns / lines, the general kernel -> here): DCT-II of
 // 300 points 1.2 / 1.3 -> 3.9 / 3.7 TB/s, DCT-I 0.9 / 0.9 -> 2.8 / 2.9, DCT-IV 0.3 /
-// 0.3 -> 3.3 / 3.5; on 513-point grids the compiled DCT-I tiles ran at 2.0 / 2.1
-// where these reach 2.5 / 2.7, the DCT-IV ones at 2.7 / 2.8 against 3.7 / 3.9.
-// What bounds the Stockham classes: up to 600 points the HBM rate of the access pattern; longer
-// columns the workgroups per CU, since a tile of 8 columns takes over half
-// of the LDS.
+// 0.3 -> 3.3 / 3.5; on 513-point grids the compiled DCT-I tiles run at 2.0 / 2.1
+// where these reach 2.5 / 2.7, the DCT-IV ones at 2.7 / 2.8 against 3.7 / 3.9 (on
+// small pencils the tiles are ahead: dtt_choice, plan.cpp).
+// What bounds the Stockham classes: up to 600 points the HBM rate of the access
+// pattern; longer columns the workgroups per CU, since a tile of 8 columns takes
+// over half of the LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
